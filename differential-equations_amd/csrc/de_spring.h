@@ -5,9 +5,28 @@
 
 #include "../../include/de_api.h"
 #include "de_lane.h"
+#include "de_spring_solvers.h"
 
 namespace de {
 namespace parity {
+
+// Size classes: systems of at most kCaps[k] masses.
+constexpr int kCaps[] = {4, 8, 16, 32, 64, 128, 256};
+constexpr int kNumCaps = 7;
+
+typedef void (*GroupKernel)(SpringArgs);
+
+// The group kernels of a method other than DOPRI5 (final state and t_eval
+// output), one shape per size class.
+struct ClassKernel {
+  int g;  // lanes per system
+  GroupKernel k;
+};
+// Translation unit `part`'s kernels of a method (kNumCaps entries), or null.
+#define DE_SPRING_PARTS(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6)
+#define DE_SPRING_PART_DECL(n) const ClassKernel* spring_method_part##n(int method);
+DE_SPRING_PARTS(DE_SPRING_PART_DECL)
+#undef DE_SPRING_PART_DECL
 
 // Launch a spring-chain ensemble.  `b` holds device pointers; host_sizes is a
 // host copy of b->sizes (the launcher buckets systems by size).  Returns 0 on

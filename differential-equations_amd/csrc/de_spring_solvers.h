@@ -10,20 +10,27 @@
 //                 an HBM workspace.  The error norm is the reference's
 //                 sequential sum, so results are bit-identical to the CPU
 //                 restatement.  The t_eval output and the point outputs.
-//   GroupDopri5   G lanes per system, C masses per lane held in registers.
-//                 Neighbour displacements cross lanes by DPP wavefront shifts
-//                 and the norms are fixed butterfly reductions (DPP within a
-//                 row, permutes across rows), identical on every lane of the
-//                 group.  The butterfly sums in a different order
+//   Group*        G lanes per system, C masses per lane held in registers.
+//                 Neighbour displacements cross lanes by DPP wavefront shifts.
+//                 GroupDopri5's norms are fixed butterfly reductions (DPP
+//                 within a row, permutes across rows), identical on every lane
+//                 of the group; the butterfly sums in a different order
 //                 than the reference's sequential loop (traits.rs:398-409), so
-//                 results agree to rounding rather than bit for bit.  DOPRI5
-//                 with the t_eval output or a point output, and event solouts.
+//                 its results agree to rounding rather than bit for bit.  The
+//                 other methods' group solvers (de_spring_group.h) keep the
+//                 one-lane solvers' bits.  GroupDopri5 has every output and
+//                 event solout, the others the final state and t_eval output.
 #pragma once
 
 #include "de_erk_tables.h"
 #include "de_lane.h"
 
 namespace de {
+
+// Blocks of the group kernels of the methods beside DOPRI5: one wavefront, so
+// that the ordered sums' LDS needs no barrier and a block that has drained
+// leaves its slot at once.
+constexpr int kGroupBlock = 64;
 
 struct SpringArgs {
   OdeArgs o;                   // common settings and per-trajectory outputs
@@ -36,7 +43,7 @@ struct SpringArgs {
   double* ev_work;             // event solouts: one state per system at state_offset
   double* ystate;              // one-lane solvers' working state at state_offset, or
                                // null: y_final (which the result then needs no copy to)
-  const int32_t* list;         // GroupDopri5: system indices of this size class
+  const int32_t* list;         // group solvers: system indices of this size class
   int64_t list_len;
 };
 
@@ -1230,10 +1237,10 @@ struct VecErk : VecCommon {
 };
 
 #if defined(__HIP_DEVICE_COMPILE__) || defined(__HIPCC__)
-// ----------------------------------------------------------- GroupDopri5 --
-// G lanes per system (G a power of two <= 64), C masses per lane:
-// lane l of the group owns masses j = l*C + q, q < C, and keeps x_j, v_j of
-// every vector in registers.
+// ----------------------------------------------------------- GroupCommon --
+// Shared pieces of the group solvers: G lanes per system (G a power of two
+// <= 64), C masses per lane: lane l of the group owns masses j = l*C + q,
+// q < C, and keeps x_j, v_j of every vector in registers.
 // A double moved across lanes by one DPP operation on each half (dpp_ctrl
 // CTRL; a lane whose source is out of range or inactive reads 0).  Lane
 // exchanges within a row and wavefront shifts are VALU operations, without
@@ -1254,8 +1261,10 @@ constexpr int kDppWaveShl1 = 0x130;   // wave_shl:1: lane i reads lane i + 1
 
 // OUT: the point outputs and event solouts are compiled in (their paths
 // would otherwise raise the register count of every group kernel).
-template <int G, int C, bool OUT = false>
-struct GroupDopri5 {
+template <int G, int C, bool OUT>
+struct GroupCommon {
+  static constexpr int kG = G, kC = C;
+  static constexpr bool kOut = OUT;
   double x[C], v[C];      // y
   double k0x[C], k0v[C];  // f(t, y)
   double kk[C + 1];       // springs k_{lC} .. k_{lC+C}
@@ -1265,9 +1274,8 @@ struct GroupDopri5 {
   double t, h, h_prev, tf, dir, rtol, atol;
   double last;  // EvenSolout::last_output_t
   double ev_value, ev_last, ev_new, tail;  // event solouts (as VecCommon's)
-  int32_t acc, rej, ev, steps, stiff, nonstiff, countdown, next_eval, pushed;
+  int32_t next_eval, pushed;
   int32_t ev_count, ev_pushed;
-  bool rejected_last;
 
   // Tolerances of state component c (x_j: c = j, v_j: c = nm + j); the
   // per-component arrays are read where used (their pointer is uniform).
@@ -1319,7 +1327,7 @@ struct GroupDopri5 {
     }
   }
 
-  DE_DEV void finish(const SpringArgs& A, int32_t st) const {
+  DE_DEV void write(const SpringArgs& A, int32_t st, int64_t acc, int64_t rej, int64_t ev) const {
     const OdeArgs& a = A.o;
     write_state(a.y_final + so, x, v);
     if (l == 0) {
@@ -1562,8 +1570,8 @@ struct GroupDopri5 {
     return true;
   }
 
-  // Load system `s`; returns false (after writing results) on BadInput.
-  DE_DEV bool init(const SpringArgs& A, int64_t s, int lane_in_group) {
+  // Load system `s`; returns t0.
+  DE_DEV double setup(const SpringArgs& A, int64_t s, int lane_in_group) {
     const OdeArgs& a = A.o;
     l = lane_in_group;
     sys = s;
@@ -1588,11 +1596,59 @@ struct GroupDopri5 {
     rtol = a.rtol_traj ? a.rtol_traj[s] : a.rtol;
     atol = a.atol_traj ? a.atol_traj[s] : a.atol;
     t = t0;
-    acc = rej = ev = steps = 0;
     pushed = next_eval = 0;
     ev_count = ev_pushed = 0;
     tail = as_f64(kNaNBits);
     dir = signum(tf - t0);
+    return t0;
+  }
+
+  // The solout call after init: (t0, y0) of a point output, the t_eval points
+  // equal to t0, g(t0, y0).
+  DE_DEV void output_start(const SpringArgs& A) {
+    const OdeArgs& a = A.o;
+    if (OUT && a.pts_mode != kPointsNone) {
+      pts_push(A, t, x, v);
+      last = t;
+    } else if (a.n_eval > 0) {
+      emit(A, t, t, x, v, [](double, double*, double*) { return true; });
+    }
+    if constexpr (OUT) ev_start(a);
+  }
+
+  // The next t_eval point is not past t_curr (or is NaN): emit has work.
+  DE_DEV bool teval_due(const OdeArgs& a, double t_curr) const {
+    if (a.n_eval <= 0 || next_eval >= a.n_eval) return false;
+    const double te = a.t_eval[next_eval];
+    return !(dir > 0.0 ? te > t_curr : te < t_curr);
+  }
+};
+
+// The members of GroupCommon by name in a solver derived from it.
+#define DE_GROUP_MEMBERS                                                                       \
+  using B = GroupCommon<G, C, OUT>;                                                            \
+  using B::x; using B::v; using B::k0x; using B::k0v; using B::nm; using B::l; using B::sys;   \
+  using B::so; using B::t; using B::h; using B::h_prev; using B::tf; using B::dir;             \
+  using B::rtol; using B::atol; using B::rt; using B::at; using B::rhs; using B::gsum;         \
+  using B::last; using B::tail; using B::next_eval; using B::pushed; using B::ev_new;          \
+  using B::ev_last; using B::setup; using B::write; using B::emit; using B::teval_due;         \
+  using B::output_start; using B::pts_push; using B::points_step; using B::ev_pre;             \
+  using B::ev_post;
+
+// ----------------------------------------------------------- GroupDopri5 --
+template <int G, int C, bool OUT = false>
+struct GroupDopri5 : GroupCommon<G, C, OUT> {
+  DE_GROUP_MEMBERS
+  int32_t acc, rej, ev, steps, stiff, nonstiff, countdown;
+  bool rejected_last;
+
+  DE_DEV void finish(const SpringArgs& A, int32_t st) const { write(A, st, acc, rej, ev); }
+
+  // Start system `s`; returns false (after writing results) on BadInput.
+  DE_DEV bool init(const SpringArgs& A, int64_t s, int lane_in_group) {
+    const OdeArgs& a = A.o;
+    const double t0 = setup(A, s, lane_in_group);
+    acc = rej = ev = steps = 0;
     bool ok = dir == 1.0 || dir == -1.0;
     double h0 = a.h0;
     if (ok && h0 == 0.0) {
@@ -1653,13 +1709,7 @@ struct GroupDopri5 {
     stiff = nonstiff = 0;
     countdown = 100;
     rejected_last = false;
-    if (OUT && a.pts_mode != kPointsNone) {
-      pts_push(A, t, x, v);
-      last = t;
-    } else if (a.n_eval > 0) {
-      emit(A, t, t, x, v, [](double, double*, double*) { return true; });
-    }
-    if constexpr (OUT) ev_start(a);
+    output_start(A);
     return true;
   }
 
@@ -1883,6 +1933,47 @@ struct GroupDopri5 {
     return false;
   }
 };
+
+// Persistent groups: each group takes the next system of the class from the
+// counter when it finishes one (one atomic per wavefront, ballot-aggregated).
+template <class Solver>
+DE_DEV void spring_group_loop(const SpringArgs& A) {
+  constexpr int G = Solver::kG;
+  const int lane = __lane_id();
+  const int l = lane & (G - 1);
+  const int leader_lane = lane - l;
+  Solver S;
+  bool have = false;
+  bool drained = false;
+  const unsigned long long len = (unsigned long long)A.list_len;
+  for (;;) {
+    if (!drained) {
+      bool need = !have;
+      unsigned long long mask = __ballot(need && l == 0);
+      if (mask) {
+        int leader = __ffsll((long long)mask) - 1;
+        int cnt = __popcll(mask);
+        unsigned long long base = 0;
+        if (lane == leader) base = atomicAdd(A.o.counter, (unsigned long long)cnt);
+        base = __shfl(base, leader);
+        if (base + (unsigned long long)cnt >= len) drained = true;
+        if (need) {
+          unsigned long long below =
+              leader_lane == 0 ? 0ull : (mask & ((1ull << leader_lane) - 1ull));
+          unsigned long long my = base + (unsigned long long)__popcll(below);
+          if (my < len) have = S.init(A, (int64_t)A.list[my], l);
+        }
+      }
+    }
+    if (!__any(have)) {
+      if (drained) break;
+      continue;
+    }
+    if (have) {
+      if (S.advance(A)) have = false;
+    }
+  }
+}
 #endif
 
 }  // namespace de

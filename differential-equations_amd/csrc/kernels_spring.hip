@@ -2,12 +2,14 @@
 //
 // Mappings (selected by de_ode_batch.mapping):
 //   DE_MAP_LANE   one thread per system, vectors in an HBM workspace (plain
-//                 launch; bit-identical to the CPU restatement).  DOPRI5, and
-//                 the only mapping of DOP853, RK4, Euler and the embedded
-//                 family.
+//                 launch; bit-identical to the CPU restatement).
 //   DE_MAP_GROUP  G lanes per system with C masses per lane in registers.
-//   DE_MAP_AUTO   systems are bucketed into size classes (N <= 4, 8, ..., 256);
-//                 for each class an autotuner times every (G, C, block) with
+//                 DOPRI5 to rounding (its norm is summed over the lanes); the
+//                 other methods keep the one-lane solvers' bits and have one
+//                 shape per size class (kernels_spring_group.hip).
+//   DE_MAP_AUTO   as DE_MAP_GROUP.  Systems are bucketed into size classes
+//                 (N <= 4, 8, ..., 256);
+//                 for each class of DOPRI5 an autotuner times every (G, C, block) with
 //                 G*C equal to the class cap on a sample of the class and keeps
 //                 the fastest.  Classes run concurrently on their own streams,
 //                 each as a persistent kernel whose groups take the next system
@@ -72,45 +74,10 @@ static LaneSolver lane_solver(int method) {
 template <int G, int C, bool OUT>
 __global__ __launch_bounds__(kSpringBlock) __attribute__((amdgpu_waves_per_eu(C == 1 ? 3 : 2))) void
 spring_group_kernel(SpringArgs A) {
-  const int lane = __lane_id();
-  const int l = lane & (G - 1);
-  const int leader_lane = lane - l;
-  GroupDopri5<G, C, OUT> S;
-  bool have = false;
-  bool drained = false;
-  const unsigned long long len = (unsigned long long)A.list_len;
-  for (;;) {
-    if (!drained) {
-      bool need = !have;
-      unsigned long long mask = __ballot(need && l == 0);
-      if (mask) {
-        int leader = __ffsll((long long)mask) - 1;
-        int cnt = __popcll(mask);
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(A.o.counter, (unsigned long long)cnt);
-        base = __shfl(base, leader);
-        if (base + (unsigned long long)cnt >= len) drained = true;
-        if (need) {
-          unsigned long long below =
-              leader_lane == 0 ? 0ull : (mask & ((1ull << leader_lane) - 1ull));
-          unsigned long long my = base + (unsigned long long)__popcll(below);
-          if (my < len) have = S.init(A, (int64_t)A.list[my], l);
-        }
-      }
-    }
-    if (!__any(have)) {
-      if (drained) break;
-      continue;
-    }
-    if (have) {
-      if (S.advance(A)) have = false;
-    }
-  }
+  spring_group_loop<GroupDopri5<G, C, OUT>>(A);
 }
 
 __global__ void spring_zero_counter(unsigned long long* c) { *c = 0ull; }
-
-typedef void (*GroupKernel)(SpringArgs);
 
 struct Config {
   int g, c;
@@ -127,13 +94,17 @@ static const Config kConfigs[] = {
 };
 #undef DE_CFG
 static const int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-static const int kCaps[] = {4, 8, 16, 32, 64, 128, 256};
-static const int kNumCaps = 7;
 static const int kBlocks[] = {64, 256};
 
 struct Choice {
   int cfg = -1;
   int block = kSpringBlock;
+};
+
+// A class's kernel in one launch.
+struct Shape {
+  GroupKernel kernel;
+  int g, block;
 };
 
 // Process-wide state: autotune decisions per size class, streams, workspace.
@@ -178,20 +149,32 @@ static GroupKernel class_kernel(const SpringArgs& base, const Config& cf) {
   return base.o.pts_mode != kPointsNone || base.o.ev.solout != kSoloutDefault ? cf.kx : cf.k;
 }
 
+static Shape shape_of(const SpringArgs& base, const Choice& ch) {
+  return {class_kernel(base, kConfigs[ch.cfg]), kConfigs[ch.cfg].g, ch.block};
+}
+
+// The kernels of a method other than DOPRI5.
+static const ClassKernel* method_kernels(int method) {
+#define DE_SPRING_PART_TRY(n) \
+  if (const ClassKernel* k = spring_method_part##n(method)) return k;
+  DE_SPRING_PARTS(DE_SPRING_PART_TRY)
+#undef DE_SPRING_PART_TRY
+  return nullptr;
+}
+
 static int launch_class(const SpringArgs& base, const int32_t* d_list, int64_t len,
-                        int64_t work_share_blocks, const Choice& ch, unsigned long long* counter,
+                        int64_t work_share_blocks, const Shape& sh, unsigned long long* counter,
                         hipStream_t s) {
-  const Config& cf = kConfigs[ch.cfg];
   SpringArgs A = base;
   A.list = d_list;
   A.list_len = len;
   A.o.counter = counter;
-  int64_t groups_per_block = ch.block / cf.g;
+  int64_t groups_per_block = sh.block / sh.g;
   int64_t need = (len + groups_per_block - 1) / groups_per_block;
   int64_t grid = work_share_blocks < need ? work_share_blocks : need;
   if (grid < 1) grid = 1;
   hipLaunchKernelGGL(spring_zero_counter, dim3(1), dim3(1), 0, s, counter);
-  hipLaunchKernelGGL(class_kernel(base, cf), dim3((unsigned)grid), dim3(ch.block), 0, s, A);
+  hipLaunchKernelGGL(sh.kernel, dim3((unsigned)grid), dim3(sh.block), 0, s, A);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -212,7 +195,9 @@ static Choice autotune(const SpringArgs& base, int k, const int32_t* d_list, int
       ch.block = block;
       int64_t full = (int64_t)g_num_cu * blocks_per_cu(class_kernel(base, kConfigs[ci]), block);
       (void)hipEventRecord(e0, s);
-      if (launch_class(base, d_list, sample, full, ch, g_counters + kNumCaps, s) != 0) continue;
+      if (launch_class(base, d_list, sample, full, shape_of(base, ch), g_counters + kNumCaps, s) !=
+          0)
+        continue;
       (void)hipEventRecord(e1, s);
       if (hipEventSynchronize(e1) != hipSuccess) continue;
       float ms = 0.0f;
@@ -228,10 +213,14 @@ static Choice autotune(const SpringArgs& base, int k, const int32_t* d_list, int
   return best;
 }
 
-// One thread per system: DE_MAP_LANE and every method but DOPRI5 (the group
-// mapping is built for DOPRI5, with every output and event solout).
+// One thread per system: when the caller asks for it, and for the point
+// outputs and event solouts of the methods beside DOPRI5 (their group kernels
+// carry the final state and the t_eval output: with an event's root search
+// inlined around a 16-stage interpolant they do not compile in minutes).
 static bool lane_mapping(const de_ode_batch* b) {
-  return b->mapping == DE_MAP_LANE || b->method != DE_METHOD_DOPRI5;
+  return b->mapping == DE_MAP_LANE ||
+         (b->method != DE_METHOD_DOPRI5 &&
+          (b->points != DE_POINTS_NONE || b->event_solout != DE_SOLOUT_DEFAULT));
 }
 
 // Start of each system's point states in points_y (n + 1 values): the slot
@@ -355,9 +344,14 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   }
   if (pts) base.pts_ypos = (const int64_t*)((const char*)d_list + list_bytes);
   // Choose a configuration per class.
-  std::vector<Choice> choice(kNumCaps);
+  const ClassKernel* fixed = method_kernels(b->method);
+  std::vector<Shape> shape(kNumCaps);
   for (int k = 0; k < kNumCaps; ++k) {
     if (lists[k].empty()) continue;
+    if (fixed) {
+      shape[k] = {fixed[k].k, fixed[k].g, kGroupBlock};
+      continue;
+    }
     Choice ch;
     if (b->mapping == DE_MAP_GROUP && b->group_size > 0) {
       for (int ci = 0; ci < kNumConfigs; ++ci)
@@ -383,7 +377,7 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
         g_tuned[k] = ch;
       }
     }
-    choice[k] = ch;
+    shape[k] = shape_of(base, ch);
   }
   // Launch classes concurrently: the three small classes first, then the
   // others largest first.  Every class kernel gets a full-device grid (capped
@@ -403,10 +397,10 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   for (int q = 0; q < kNumCaps && ok; ++q) {
     const int k = kLaunchOrder[q];
     if (lists[k].empty()) continue;
-    const Choice& ch = choice[k];
-    int64_t share = (int64_t)g_num_cu * blocks_per_cu(class_kernel(base, kConfigs[ch.cfg]), ch.block);
+    const Shape& sh = shape[k];
+    int64_t share = (int64_t)g_num_cu * blocks_per_cu(sh.kernel, sh.block);
     ok = hipStreamWaitEvent(g_streams[k], g_fork, 0) == hipSuccess &&
-         launch_class(base, d_list + start[k], (int64_t)lists[k].size(), share, ch,
+         launch_class(base, d_list + start[k], (int64_t)lists[k].size(), share, sh,
                       g_counters + k, g_streams[k]) == 0 &&
          hipEventRecord(g_join[k], g_streams[k]) == hipSuccess &&
          hipStreamWaitEvent(s, g_join[k], 0) == hipSuccess;

@@ -1,0 +1,118 @@
+"""GPU: the spring chains' group kernels of the methods beside DOPRI5 give the
+CPU restatement's values (as the one-lane mapping does), at the sizes where a
+size class or a lane's masses end."""
+import numpy as np
+import pytest
+
+import deamd
+from deamd import DE_MAP_AUTO, DE_MAP_GROUP, DE_MAP_LANE, IVP, ExplicitRungeKutta, SpringChain
+
+pytestmark = pytest.mark.gpu
+
+THREADS = 8
+ADAPTIVE = ["dop853", "rkf45", "cash_karp", "rkv655e", "rkv656e", "rkv766e", "rkv767e", "rkv877e",
+            "rkv878e", "rkv988e", "rkv989e"]
+FIXED = ["rk4", "euler"]
+# One below, at and above every class bound, odd remainders inside the classes
+# of two and four masses per lane, and a lone mass.
+EDGES = [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 66, 95, 96, 97, 127, 128,
+         129, 130, 131, 191, 192, 193, 254, 255, 256]
+
+
+def chains(sizes, seed):
+    sizes = np.asarray(sizes, dtype=np.int32)
+    rng = np.random.default_rng(seed)
+    params, y0 = [], []
+    for n in sizes:
+        params += [rng.uniform(0.0, 0.1, 1), np.exp(0.5 * rng.standard_normal(n + 1))]
+        y0 += [rng.standard_normal(n), 0.1 * rng.standard_normal(n)]
+    return SpringChain(sizes, np.concatenate(params)), np.concatenate(y0)
+
+
+def make(method, rtol=1e-7, h=0.01):
+    M = ExplicitRungeKutta
+    if method in FIXED:
+        return getattr(M, method)(h).max_steps(200000)
+    return getattr(M, method)().rtol(rtol).atol(rtol * 1e-2).max_steps(200000)
+
+
+def check(orc, ens, mappings=(DE_MAP_AUTO,)):
+    # Equal values, NaN where the oracle has NaN; a zero's sign may differ in
+    # the embedded family, whose kernels skip zero coefficients.
+    want = orc.solve_ode(ens, threads=THREADS)
+    for mapping in mappings:
+        got = ens.options(mapping=mapping, group_size=8 if mapping == DE_MAP_GROUP else 0).solve()
+        for f in ("status", "accepted", "rejected", "evals"):
+            assert np.array_equal(getattr(got, f), getattr(want, f)), (f, mapping)
+        for f in ("t", "y", "dense", "n_dense"):
+            g, w = getattr(got, f), getattr(want, f)
+            assert (g is None) == (w is None)
+            if g is not None:
+                assert np.array_equal(g, w, equal_nan=g.dtype.kind == "f"), (f, mapping)
+    return want
+
+
+@pytest.mark.parametrize("method", ADAPTIVE + FIXED)
+def test_class_edges(orc, method):
+    sysm, y0 = chains(EDGES, 71)
+    base = lambda: IVP.ode(sysm, 0.0, 1.5, y0).method(make(method))  # noqa: E731
+    check(orc, base(), (DE_MAP_AUTO, DE_MAP_GROUP, DE_MAP_LANE))
+    # t0, the end and points off both ends among the output times.
+    check(orc, base().t_eval(np.concatenate([np.linspace(-0.2, 1.7, 17), [0.0, 1.5]])))
+
+
+@pytest.mark.parametrize("method", ["rk4", "dop853", "rkf45", "rkv767e"])
+def test_spans_tolerances_and_statuses(orc, method):
+    # Per-system spans (forward, backward, empty: BadInput), per-component and
+    # per-system tolerances, and a step limit that some systems reach.
+    rng = np.random.default_rng(72)
+    sizes = rng.integers(1, 257, 90)
+    sysm, y0 = chains(sizes, 73)
+    n, state = len(sizes), int(2 * sizes.sum())
+    t0 = rng.uniform(-1.0, 1.0, n)
+    tf = t0 + rng.uniform(0.2, 2.0, n)
+    tf[::9] = t0[::9]
+    if method not in FIXED:
+        tf[1::3] = t0[1::3] - 0.7
+    ens = IVP.ode(sysm, t0, tf, y0).method(make(method).max_steps(60))
+    ens.rtol_traj = np.where(np.arange(n) % 2 == 0, 1e-5, 1e-8)
+    ens.atol_traj = ens.rtol_traj * 1e-2
+    want = check(orc, ens, (DE_MAP_AUTO, DE_MAP_LANE))
+    assert set(want.status) >= {deamd.DE_STATUS_COMPLETE, deamd.DE_STATUS_BAD_INPUT}
+    ens.rtol_comp = 10.0 ** rng.uniform(-8, -5, state)
+    ens.atol_comp = ens.rtol_comp * 1e-2
+    check(orc, ens)
+    # Backward with output: the solve ends at its first interior point.
+    back = IVP.ode(sysm, 0.0, -1.0 if method not in FIXED else 1.0, y0).method(
+        make(method)).t_eval(np.linspace(0.0, -1.0, 5) if method not in FIXED else [0.5])
+    check(orc, back)
+
+
+@pytest.mark.parametrize("method", ["dop853", "rkf45", "rkv877e"])
+def test_values_that_overflow(orc, method):
+    # Springs stiff enough that stages overflow: rejections, NaN where the
+    # reference's combinations give NaN, and the stiffness and step-size ends.
+    sysm, y0 = chains([1, 4, 5, 33, 64, 65, 129, 200], 74)
+    p = sysm.params_packed.copy()
+    for i in range(0, len(sysm.sizes), 2):
+        lo = int(sysm.param_offset[i])
+        p[lo + 1:lo + 2 + int(sysm.sizes[i])] = 1e200
+    y0 = y0.copy()
+    y0[-3] = np.inf
+    ens = IVP.ode(SpringChain(sysm.sizes, p), 0.0, 1.0, y0).method(
+        make(method).h0(0.1).max_steps(500).max_rejects(7))
+    check(orc, ens, (DE_MAP_AUTO, DE_MAP_LANE))
+
+
+def test_results_do_not_depend_on_the_batch(orc):
+    # A system alone and among others gives the same bits.
+    sysm, y0 = chains([6, 40, 100, 200, 6, 40, 100, 200, 3], 75)
+    for method in ("dop853", "rkv656e", "rk4"):
+        whole = IVP.ode(sysm, 0.0, 2.0, y0).method(make(method)).solve()
+        for i in (2, 3, 8):
+            a, b = int(sysm.state_offset[i]), int(sysm.state_offset[i + 1])
+            pa, pb = int(sysm.param_offset[i]), int(sysm.param_offset[i + 1])
+            one = IVP.ode(SpringChain(sysm.sizes[i:i + 1], sysm.params_packed[pa:pb]), 0.0, 2.0,
+                          y0[a:b]).method(make(method)).solve()
+            assert np.array_equal(one.y, whole.y[a:b])
+            assert one.accepted[0] == whole.accepted[i] and one.evals[0] == whole.evals[i]
