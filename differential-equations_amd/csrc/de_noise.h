@@ -19,13 +19,6 @@ namespace de {
 
 DE_TABLE double kNoiseLogTable[128 * 2] = DE_NOISE_LOG_TABLE;
 
-// Nearest integer of v (ties to even) for |v| < 2^51, with exact operations.
-DE_HD double round_to_int(double v) {
-  DE_NO_CONTRACT
-  const double shift = 0x1.8p52;
-  return (v + shift) - shift;
-}
-
 struct u32x4 {
   uint32_t v[4];
 };
@@ -56,6 +49,91 @@ DE_HD u32x4 philox4x32_10(u32x4 ctr, uint32_t k0, uint32_t k1) {
     ctr = n;
   }
   return ctr;
+}
+
+// a ^ b ^ c, one instruction on gfx950 (a truth-table operation on three words).
+DE_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
+// The Philox4x32-10 blocks (j, step, path), j < NB, of one path: the words of
+// the first three rounds that do not depend on the step are formed once per
+// path, and the one first-round product that depends on the step but not on j
+// once per step.  What is left per step is 1 product for all blocks and 15 per
+// block instead of 20 per block, each with one three-input exclusive or.
+template <int NB>
+struct PhiloxPath {
+  uint32_t n0;         // round 1: word 0 without the step
+  uint32_t p1k[NB];    // round 2: word 1 ^ round 3's key 0
+  uint32_t c0h[NB];    // round 3: high half of the first product ^ key 1
+  uint32_t c0l[NB];    // round 3: word 3 ^ round 4's key 1
+
+  DE_HD static constexpr uint32_t key0(uint32_t k, int round) {
+    return k + (uint32_t)round * 0x9E3779B9u;
+  }
+  DE_HD static constexpr uint32_t key1(uint32_t k, int round) {
+    return k + (uint32_t)round * 0xBB67AE85u;
+  }
+  static constexpr uint32_t kM0 = 0xD2511F53u, kM1 = 0xCD9E8D57u;
+
+  DE_HD void start(uint64_t path, uint32_t k0, uint32_t k1) {
+    uint32_t hi, lo;
+    mulhilo32(kM1, (uint32_t)path, &hi, &lo);
+    n0 = hi ^ k0;
+    const uint32_t n1 = lo;
+    for (int j = 0; j < NB; ++j) {
+      const uint64_t m0j = (uint64_t)kM0 * (uint32_t)j;
+      const uint32_t n2 = (uint32_t)(m0j >> 32) ^ (uint32_t)(path >> 32) ^ k1;
+      mulhilo32(kM1, n2, &hi, &lo);
+      const uint32_t p0 = hi ^ n1 ^ key0(k0, 1);
+      p1k[j] = lo ^ key0(k0, 2);
+      mulhilo32(kM0, p0, &hi, &lo);
+      c0h[j] = hi ^ key1(k1, 2);
+      c0l[j] = lo ^ key1(k1, 3);
+    }
+  }
+  // The step's shared product.
+  DE_HD void step(uint32_t call, uint32_t* hi, uint32_t* lo) const {
+    mulhilo32(kM0, n0 ^ call, hi, lo);
+  }
+  DE_HD u32x4 block(int j, uint32_t step_hi, uint32_t step_lo, uint32_t k0, uint32_t k1) const {
+    uint32_t hi0, lo0, hi1, lo1;
+    const uint32_t m0j = (uint32_t)((uint64_t)kM0 * (uint32_t)j);
+    mulhilo32(kM1, step_hi ^ (m0j ^ key1(k1, 1)), &hi1, &lo1);
+    uint32_t c0 = hi1 ^ p1k[j], c1 = lo1, c2 = c0h[j] ^ step_lo, c3;
+    // Round 4, whose key 1 is in c0l already.
+    mulhilo32(kM0, c0, &hi0, &lo0);
+    mulhilo32(kM1, c2, &hi1, &lo1);
+    c0 = xor3(hi1, c1, key0(k0, 3));
+    c1 = lo1;
+    c2 = hi0 ^ c0l[j];
+    c3 = lo0;
+#pragma unroll
+    for (int round = 4; round < 10; ++round) {
+      mulhilo32(kM0, c0, &hi0, &lo0);
+      mulhilo32(kM1, c2, &hi1, &lo1);
+      c0 = xor3(hi1, c1, key0(k0, round));
+      c1 = lo1;
+      c2 = xor3(hi0, c3, key1(k1, round));
+      c3 = lo0;
+    }
+    return u32x4{{c0, c1, c2, c3}};
+  }
+};
+
+// x with its sign flipped where bit 31 of `bit` is set.
+DE_HD double flip_sign(double x, uint32_t bit) {
+  const uint64_t u = as_u64(x);
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(u >> 32), bit, 0x80000000u, 0x78);
+#else
+  const uint32_t hi = (uint32_t)(u >> 32) ^ (bit & 0x80000000u);
+#endif
+  return as_f64(((uint64_t)hi << 32) | (uint32_t)u);
 }
 
 // fma(a, b, c) as one three-operand instruction on the device.  With c a
@@ -158,21 +236,26 @@ DE_HD double noise_sqrt(double x) {
 // Two independent standard normals from one Philox block (Box-Muller).
 // Angle 2*pi*u2 is reduced in quarter turns, which is exact.
 DE_HD void box_muller(u32x4 w, double* z0, double* z1) {
+  DE_NO_CONTRACT
   double u1 = uniform_oc(w.v[0], w.v[1]);
-  double u2 = uniform_co(w.v[2], w.v[3]);
   double rad = noise_sqrt(-2.0 * noise_log(u1));   // 0 or >= 2^-52
-  double q4 = 4.0 * u2;
-  double qd = round_to_int(q4);
+  // q4 = 4 u2 with u2 = uniform_co(w.v[2], w.v[3]), exact like u2.
+  const double q4 = fma((double)(w.v[3] >> 11), 0x1p-51, (double)w.v[2] * 0x1p-30);
+  // The nearest integer of q4 (ties to even, exact operations): the sum's low
+  // word is that integer, so the quarter needs no conversion.
+  const double qs = q4 + 0x1.8p52;
+  const double qd = qs - 0x1.8p52;
+  const uint32_t q = (uint32_t)as_u64(qs);
   double f = q4 - qd;                            // [-0.5, 0.5], exact
   double th = f * DE_NOISE_HALF_PI;
   double s, c;
   noise_sincos_small(th, &s, &c);
-  // Quarter q: (cos, sin) = (c, s), (-s, c), (-c, -s), (s, -c).
-  const int q = ((int)qd) & 3;
-  const double a = (q & 1) ? s : c;
-  const double b = (q & 1) ? c : s;
-  *z0 = rad * (((q + 1) & 2) ? -a : a);
-  *z1 = rad * ((q & 2) ? -b : b);
+  // Quarter q: (cos, sin) = (c, s), (-s, c), (-c, -s), (s, -c): swapped for
+  // odd q, the signs from bit 1 of q + 1 and of q.
+  const double a = (q & 1u) ? s : c;
+  const double b = (q & 1u) ? c : s;
+  *z0 = rad * flip_sign(a, (q + 1u) << 30);
+  *z1 = rad * flip_sign(b, q << 30);
 }
 
 // Standard normal for (seed, path, step, component).  Components 2j and 2j+1

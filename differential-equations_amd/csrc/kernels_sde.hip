@@ -25,17 +25,27 @@ struct SdeLane {
   double y[D], dydt[D];
   double t, h, tf, dir;
   int64_t steps, ev;
-  uint64_t path;
-  double sqrt_h;  // sqrt(h), formed where h is set (the start and the clipped last step)
+  PhiloxPath<(D + 1) / 2> noise;
+  // sqrt(h) and Milstein's 1 / (2 sqrt(h)), formed where h is set (the start
+  // and the clipped last step).
+  double sqrt_h, factor;
+
+  DE_DEV void set_h(double hh) {
+    h = hh;
+    sqrt_h = sqrt(h);
+    factor = 1.0 / (2.0 * sqrt_h);
+  }
 
   DE_DEV void noise_fill(const SdeArgs& a, double* dw) const {
     uint32_t call = (uint32_t)(steps - 1);
     if (a.noise == kNoisePhilox) {
       const double sq = sqrt_h;
+      uint32_t step_hi, step_lo;
+      noise.step(call, &step_hi, &step_lo);
 #pragma unroll
       for (int c = 0; c < D; c += 2) {
-        u32x4 ctr = {{(uint32_t)(c >> 1), call, (uint32_t)path, (uint32_t)(path >> 32)}};
-        u32x4 w = philox4x32_10(ctr, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
+        const u32x4 w = noise.block(c >> 1, step_hi, step_lo, (uint32_t)a.seed,
+                                    (uint32_t)(a.seed >> 32));
         double z0, z1;
         box_muller(w, &z0, &z1);
         dw[c] = sq * z0;
@@ -60,7 +70,8 @@ struct SdeLane {
   template <int SCHEME>
   DE_DEV void run(const SdeArgs& a, int64_t i) {
     sys.load(a.params, a.n, i);
-    path = a.path_base + (uint64_t)i;
+    if (a.noise == kNoisePhilox)
+      noise.start(a.path_base + (uint64_t)i, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
     for (int c = 0; c < D; ++c) y[c] = a.y0[(int64_t)c * a.n + i];
     t = a.t0;
     tf = a.tf;
@@ -76,16 +87,14 @@ struct SdeLane {
       finish(a, i, 0, kBadInput);
       return;
     }
-    h = h0;
-    sqrt_h = sqrt(h);
+    set_h(h0);
     sys.drift(t, y, dydt);
     ev = SCHEME == kSchemeMilstein ? 1 : 2;  // EM init also evaluates the diffusion
     for (;;) {
       if ((t + h - tf) * dir > 0.0) {
         double hn = tf - t;
         if (fabs(hn) < kTenEps) break;
-        h = hn;
-        sqrt_h = sqrt(h);
+        set_h(hn);
       }
       if (steps >= a.max_steps) {
         finish(a, i, acc, kMaxSteps);
@@ -107,7 +116,6 @@ struct SdeLane {
         double yaux[D], baux[D];
         for (int c = 0; c < D; ++c) yaux[c] = y[c] + sqrt_h * b[c];
         sys.diffusion(t, yaux, baux);
-        double factor = 1.0 / (2.0 * sqrt_h);
         for (int c = 0; c < D; ++c) {
           double term = (baux[c] - b[c]) * (dw[c] * dw[c] - h) * factor;
           ynext[c] = ((y[c] + dydt[c] * h) + b[c] * dw[c]) + term;
@@ -132,8 +140,19 @@ struct SdeLane {
 
 constexpr int kSdeBlock = 256;
 
+// Bound: VALU issue.  OU-8 Euler-Maruyama, 1 M paths x 1000 steps: 15.6 ms
+// (67 G path-steps/s) with PhiloxPath's blocks and the three-input exclusive or,
+// 20.7 ms with a rolled Philox loop per block; geometric Brownian motion with
+// Milstein 4.04 against 5.09 ms (1 M paths x 1000 steps), its 1 / (2 sqrt(h))
+// formed with h.  The polynomials' coefficients read from scalar registers fit
+// a fourth wave per SIMD at eight components, but their spills cost more (16.3
+// ms).  Milstein at eight components is held to the 168 registers of three waves
+// per SIMD (4.32 against 4.60 ms, 0.5 M paths x 500 steps); Euler-Maruyama, which
+// takes 163 by itself, schedules worse under that hint (15.8 ms).
 template <class S, int SCHEME>
-__global__ __launch_bounds__(kSdeBlock) void sde_kernel(SdeArgs a) {
+__global__ __launch_bounds__(kSdeBlock)
+__attribute__((amdgpu_waves_per_eu(SCHEME == kSchemeMilstein && S::kDim == 8 ? 3 : 1))) void
+sde_kernel(SdeArgs a) {
   int64_t i = (int64_t)blockIdx.x * kSdeBlock + threadIdx.x;
   if (i >= a.n) return;
   SdeLane<S> L;
