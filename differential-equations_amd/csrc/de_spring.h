@@ -34,8 +34,8 @@ DE_SPRING_PARTS(DE_SPRING_PART_DECL)
 int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArgs& a, int sched,
                   hipStream_t s);
 int64_t spring_workspace_bytes(const de_ode_batch* b);
-// Autotuner decision for the size class with cap masses: 0 and (G, C, block),
-// or -1 if that class has not been tuned in this process.
+// The library's shape for the size class with cap masses: 0 and (G, C, block), or
+// -1 if none of its systems has been solved in this process.
 int spring_tuned(int cap, int* g, int* c, int* block);
 
 }  // namespace parity

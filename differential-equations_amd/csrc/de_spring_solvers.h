@@ -1252,12 +1252,41 @@ DE_DEV double dpp_double(double x) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
   return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
 }
+// The same, lanes without a source reading 0 without a register set up for it.
+template <int CTRL>
+DE_DEV double dpp_double_or0(double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+// A value and that of the lane whose index differs in bit 4 or 5 (SWAP = 16,
+// 32), in an order that is the same on both lanes: the row or half exchange of
+// gfx950, a VALU operation (a permute goes through LDS).
+template <int SWAP>
+DE_DEV void swap_pair(double x, double* a, double* b) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const unsigned lo = (unsigned)u, hi = (unsigned)(u >> 32);
+  if constexpr (SWAP == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    *a = __longlong_as_double((long long)(((uint64_t)h[0] << 32) | l[0]));
+    *b = __longlong_as_double((long long)(((uint64_t)h[1] << 32) | l[1]));
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    *a = __longlong_as_double((long long)(((uint64_t)h[0] << 32) | l[0]));
+    *b = __longlong_as_double((long long)(((uint64_t)h[1] << 32) | l[1]));
+  }
+}
 constexpr int kDppQuadSwap1 = 0xB1;   // quad_perm [1,0,3,2]: lane i reads i ^ 1
 constexpr int kDppQuadSwap2 = 0x4E;   // quad_perm [2,3,0,1]: lane i reads i ^ 2
 constexpr int kDppHalfMirror = 0x141; // row_half_mirror: lane i reads 7 - i in its 8
 constexpr int kDppMirror = 0x140;     // row_mirror: lane i reads 15 - i in its 16
 constexpr int kDppWaveShr1 = 0x138;   // wave_shr:1: lane i reads lane i - 1
 constexpr int kDppWaveShl1 = 0x130;   // wave_shl:1: lane i reads lane i + 1
+constexpr int kDppRowShr1 = 0x111;    // row_shr:1: the same within a row of 16 lanes
+constexpr int kDppRowShl1 = 0x101;    // row_shl:1
 
 // OUT: the point outputs and event solouts are compiled in (their paths
 // would otherwise raise the register count of every group kernel).
@@ -1282,6 +1311,17 @@ struct GroupCommon {
   DE_DEV double rt(const OdeArgs& a, int c) const { return a.rtol_comp ? a.rtol_comp[so + c] : rtol; }
   DE_DEV double at(const OdeArgs& a, int c) const { return a.atol_comp ? a.atol_comp[so + c] : atol; }
 
+  // Sum of a lane's terms in pairs.  With gsum's levels this is one tree over the
+  // mass index for every power-of-two shape (G, C), whose zero terms beyond N add
+  // nothing: a system's sums do not depend on the shape the autotuner picks.
+  // (Three masses per lane are a tree of their own, in classes of their own.)
+  DE_DEV static double lane_sum(const double* e) {
+    if constexpr (C == 1) return e[0];
+    if constexpr (C == 2) return e[0] + e[1];
+    if constexpr (C == 3) return (e[0] + e[1]) + e[2];
+    if constexpr (C == 4) return (e[0] + e[1]) + (e[2] + e[3]);
+  }
+
   // Sum over the group's G lanes, identical on every lane: each level adds
   // the value of a partner lane under an involution (xor 1, xor 2, the mirror
   // within 8 and within 16, then xor 16 and xor 32), so a lane and its partner
@@ -1291,28 +1331,50 @@ struct GroupCommon {
     if constexpr (G >= 4) s += dpp_double<kDppQuadSwap2>(s);
     if constexpr (G >= 8) s += dpp_double<kDppHalfMirror>(s);
     if constexpr (G >= 16) s += dpp_double<kDppMirror>(s);
-    if constexpr (G >= 32) s += __shfl_xor(s, 16, G);
-    if constexpr (G >= 64) s += __shfl_xor(s, 32, G);
+    double a, b;
+    if constexpr (G >= 32) {
+      swap_pair<16>(s, &a, &b);
+      s = a + b;
+    }
+    if constexpr (G >= 64) {
+      swap_pair<32>(s, &a, &b);
+      s = a + b;
+    }
     return s;
   }
 
+  // The neighbours' displacements xs[C - 1] of lane l - 1 and xs[0] of lane
+  // l + 1, 0 beyond the group (the chain's fixed ends): a shift within a row or
+  // the whole wavefront leaves 0 at its ends, the other groups select it.
+  DE_DEV void neighbours(const double* xs, double* left, double* right) const {
+    if constexpr (G == 16) {
+      *left = dpp_double_or0<kDppRowShr1>(xs[C - 1]);
+      *right = dpp_double_or0<kDppRowShl1>(xs[0]);
+    } else {
+      *left = dpp_double_or0<kDppWaveShr1>(xs[C - 1]);
+      *right = dpp_double_or0<kDppWaveShl1>(xs[0]);
+      if constexpr (G != 64) {
+        *left = l == 0 ? 0.0 : *left;
+        *right = l == G - 1 ? 0.0 : *right;
+      }
+    }
+  }
+
   // (dx, dv) = f(x, v): dx_j = v_j, dv_j = spring_accel(...), zero beyond N.
-  // The neighbours' displacements come by a wavefront shift; a group's first
-  // and last lanes take the chain's fixed ends instead.
   DE_DEV void rhs(const double* xs, const double* vs, double* dx, double* dv) const {
-    double left = dpp_double<kDppWaveShr1>(xs[C - 1]);
-    double right = dpp_double<kDppWaveShl1>(xs[0]);
-    if (l == 0) left = 0.0;
-    if (l == G - 1) right = 0.0;
+    double left, right;
+    neighbours(xs, &left, &right);
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       const int j = l * C + q;
       double xm = q == 0 ? left : xs[q - 1];
       double xp = q == C - 1 ? right : xs[q + 1];
-      if (j + 1 >= nm) xp = 0.0;
-      bool real = j < nm;
+      xp = j + 1 >= nm ? 0.0 : xp;
+      const bool real = j < nm;
+      // Evaluated on every lane: a branch around seven operations costs more.
+      const double acc = spring_accel(xm, xs[q], xp, vs[q], kk[q], kk[q + 1], cd);
       dx[q] = real ? vs[q] : 0.0;
-      dv[q] = real ? spring_accel(xm, xs[q], xp, vs[q], kk[q], kk[q + 1], cd) : 0.0;
+      dv[q] = real ? acc : 0.0;
     }
   }
 
@@ -1630,12 +1692,22 @@ struct GroupCommon {
   using B::x; using B::v; using B::k0x; using B::k0v; using B::nm; using B::l; using B::sys;   \
   using B::so; using B::t; using B::h; using B::h_prev; using B::tf; using B::dir;             \
   using B::rtol; using B::atol; using B::rt; using B::at; using B::rhs; using B::gsum;         \
+  using B::lane_sum;                                                                           \
   using B::last; using B::tail; using B::next_eval; using B::pushed; using B::ev_new;          \
   using B::ev_last; using B::setup; using B::write; using B::emit; using B::teval_due;         \
   using B::output_start; using B::pts_push; using B::points_step; using B::ev_pre;             \
-  using B::ev_post;
+  using B::ev_post; using B::kk; using B::cd; using B::neighbours;
 
 // ----------------------------------------------------------- GroupDopri5 --
+// Bound: FP64 VALU.  Masses beyond N are cleared by selects, since branches
+// around them cut the step into pieces that could not be scheduled together.
+// The step's sums keep the reference's roundings: the error estimate cancels, so
+// that fused products in them (8.1 against 8.5 ms) move the first steps' sizes by
+// 1e-10 and, with them, the end of a solve that ends before tf.  The interpolant,
+// which nothing depends on, is fused.  65 536 chains of 4 to 256 masses, t in
+// [0, 10], 100 output times: 8.5 ms, of 11.7 with branches around the masses
+// beyond N, exchanges across rows through LDS and size classes of powers of two
+// only.
 template <int G, int C, bool OUT = false>
 struct GroupDopri5 : GroupCommon<G, C, OUT> {
   DE_GROUP_MEMBERS
@@ -1643,6 +1715,22 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
   bool rejected_last;
 
   DE_DEV void finish(const SpringArgs& A, int32_t st) const { write(A, st, acc, rej, ev); }
+
+  // rhs with fewer selects: a lane's masses beyond N stay at x = v = 0, so that
+  // the last mass finds the fixed end there and only their acceleration (the
+  // last spring's pull) is cleared.
+  DE_DEV void rhs0(const double* xs, const double* vs, double* dx, double* dv) const {
+    double left, right;
+    neighbours(xs, &left, &right);
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+      const double xm = q == 0 ? left : xs[q - 1];
+      const double xp = q == C - 1 ? right : xs[q + 1];
+      const double acc = spring_accel(xm, xs[q], xp, vs[q], kk[q], kk[q + 1], cd);
+      dx[q] = vs[q];
+      dv[q] = l * C + q < nm ? acc : 0.0;
+    }
+  }
 
   // Start system `s`; returns false (after writing results) on BadInput.
   DE_DEV bool init(const SpringArgs& A, int64_t s, int lane_in_group) {
@@ -1654,23 +1742,23 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
     if (ok && h0 == 0.0) {
       double f0x[C], f0v[C], skx[C], skv[C], y1x[C], y1v[C], f1x[C], f1v[C];
       rhs(x, v, f0x, f0v);
-      double dnf = 0.0, dny = 0.0;
+      double en[C], ey[C];
 #pragma unroll
       for (int q = 0; q < C; ++q) {
+        en[q] = ey[q] = 0.0;
         if (l * C + q < nm) {
           const int j = l * C + q;
           skx[q] = at(a, j) + rt(a, j) * fabs(x[q]);
           skv[q] = at(a, nm + j) + rt(a, nm + j) * fabs(v[q]);
           double u = f0x[q] / skx[q], u2 = f0v[q] / skv[q];
-          dnf += u * u + u2 * u2;
+          en[q] = u * u + u2 * u2;
           double w = x[q] / skx[q], w2 = v[q] / skv[q];
-          dny += w * w + w2 * w2;
+          ey[q] = w * w + w2 * w2;
         } else {
           skx[q] = skv[q] = 1.0;
         }
       }
-      dnf = gsum(dnf);
-      dny = gsum(dny);
+      const double dnf = gsum(lane_sum(en)), dny = gsum(lane_sum(ey));
       double hh = (dnf <= 1.0e-10 || dny <= 1.0e-10) ? 1.0e-6 : sqrt(dny / dnf) * 0.01;
       hh = fmin(hh, a.h_max);
       hh *= dir;
@@ -1680,15 +1768,15 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
         y1v[q] = v[q] + hh * f0v[q];
       }
       rhs(y1x, y1v, f1x, f1v);
-      double der2 = 0.0;
 #pragma unroll
       for (int q = 0; q < C; ++q) {
+        en[q] = 0.0;
         if (l * C + q < nm) {
           double d = (f1x[q] - f0x[q]) / skx[q], d2 = (f1v[q] - f0v[q]) / skv[q];
-          der2 += d * d + d2 * d2;
+          en[q] = d * d + d2 * d2;
         }
       }
-      der2 = sqrt(gsum(der2)) / fabs(hh);
+      const double der2 = sqrt(gsum(lane_sum(en))) / fabs(hh);
       double der12 = fmax(sqrt(dnf), der2);
       double h1 = der12 <= 1.0e-15 ? fabs(hh) * 1.0e-3 : DE_CTRL_POW(0.01 / der12, 1.0 / 5.0);
       double interval = fabs(tf - t0);
@@ -1745,75 +1833,61 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
       sx[q] = x[q] + a10h * k0x[q];
       sv[q] = v[q] + a10h * k0v[q];
     }
-    rhs(sx, sv, k1x, k1v);
+    rhs0(sx, sv, k1x, k1v);
     const double a20h = dp::a20 * h, a21h = dp::a21 * h;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       sx[q] = (x[q] + a20h * k0x[q]) + a21h * k1x[q];
       sv[q] = (v[q] + a20h * k0v[q]) + a21h * k1v[q];
     }
-    rhs(sx, sv, k2x, k2v);
+    rhs0(sx, sv, k2x, k2v);
     const double a30h = dp::a30 * h, a31h = dp::a31 * h, a32h = dp::a32 * h;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       sx[q] = ((x[q] + a30h * k0x[q]) + a31h * k1x[q]) + a32h * k2x[q];
       sv[q] = ((v[q] + a30h * k0v[q]) + a31h * k1v[q]) + a32h * k2v[q];
     }
-    rhs(sx, sv, k3x, k3v);
-    const double a40h = dp::a40 * h, a41h = dp::a41 * h, a42h = dp::a42 * h,
-                 a43h = dp::a43 * h;
+    rhs0(sx, sv, k3x, k3v);
+    const double a40h = dp::a40 * h, a41h = dp::a41 * h, a42h = dp::a42 * h, a43h = dp::a43 * h;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       sx[q] = (((x[q] + a40h * k0x[q]) + a41h * k1x[q]) + a42h * k2x[q]) + a43h * k3x[q];
       sv[q] = (((v[q] + a40h * k0v[q]) + a41h * k1v[q]) + a42h * k2v[q]) + a43h * k3v[q];
     }
-    rhs(sx, sv, k4x, k4v);
-    const double a50h = dp::a50 * h, a51h = dp::a51 * h, a52h = dp::a52 * h,
-                 a53h = dp::a53 * h, a54h = dp::a54 * h;
+    rhs0(sx, sv, k4x, k4v);
+    const double a50h = dp::a50 * h, a51h = dp::a51 * h, a52h = dp::a52 * h, a53h = dp::a53 * h, a54h = dp::a54 * h;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
-      sx[q] = ((((x[q] + a50h * k0x[q]) + a51h * k1x[q]) + a52h * k2x[q]) + a53h * k3x[q]) +
-              a54h * k4x[q];
-      sv[q] = ((((v[q] + a50h * k0v[q]) + a51h * k1v[q]) + a52h * k2v[q]) + a53h * k3v[q]) +
-              a54h * k4v[q];
+      sx[q] = ((((x[q] + a50h * k0x[q]) + a51h * k1x[q]) + a52h * k2x[q]) + a53h * k3x[q]) + a54h * k4x[q];
+      sv[q] = ((((v[q] + a50h * k0v[q]) + a51h * k1v[q]) + a52h * k2v[q]) + a53h * k3v[q]) + a54h * k4v[q];
     }
-    rhs(sx, sv, k5x, k5v);
-    const double a60h = dp::a60 * h, a62h = dp::a62 * h, a63h = dp::a63 * h,
-                 a64h = dp::a64 * h, a65h = dp::a65 * h;
+    rhs0(sx, sv, k5x, k5v);
+    const double a60h = dp::a60 * h, a62h = dp::a62 * h, a63h = dp::a63 * h, a64h = dp::a64 * h, a65h = dp::a65 * h;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
-      sx[q] = ((((x[q] + a60h * k0x[q]) + a62h * k2x[q]) + a63h * k3x[q]) + a64h * k4x[q]) +
-              a65h * k5x[q];
-      sv[q] = ((((v[q] + a60h * k0v[q]) + a62h * k2v[q]) + a63h * k3v[q]) + a64h * k4v[q]) +
-              a65h * k5v[q];
+      sx[q] = ((((x[q] + a60h * k0x[q]) + a62h * k2x[q]) + a63h * k3x[q]) + a64h * k4x[q]) + a65h * k5x[q];
+      sv[q] = ((((v[q] + a60h * k0v[q]) + a62h * k2v[q]) + a63h * k3v[q]) + a64h * k4v[q]) + a65h * k5v[q];
     }
-    rhs(sx, sv, k6x, k6v);
-    double segx[C], segv[C], nx[C], nv[C];
-    double err = 0.0;
+    rhs0(sx, sv, k6x, k6v);
+    double segx[C], segv[C], nx[C], nv[C], en[C];
 #pragma unroll
     for (int q = 0; q < C; ++q) {
-      segx[q] = (((dp::b0 * k0x[q] + dp::b2 * k2x[q]) + dp::b3 * k3x[q]) + dp::b4 * k4x[q]) +
-                dp::b5 * k5x[q];
-      segv[q] = (((dp::b0 * k0v[q] + dp::b2 * k2v[q]) + dp::b3 * k3v[q]) + dp::b4 * k4v[q]) +
-                dp::b5 * k5v[q];
+      segx[q] = (((dp::b0 * k0x[q] + dp::b2 * k2x[q]) + dp::b3 * k3x[q]) + dp::b4 * k4x[q]) + dp::b5 * k5x[q];
+      segv[q] = (((dp::b0 * k0v[q] + dp::b2 * k2v[q]) + dp::b3 * k3v[q]) + dp::b4 * k4v[q]) + dp::b5 * k5v[q];
       nx[q] = x[q] + h * segx[q];
       nv[q] = v[q] + h * segv[q];
-      if (l * C + q < nm) {
-        double ex = ((((dp::e0 * k0x[q] + dp::e2 * k2x[q]) + dp::e3 * k3x[q]) +
-                      dp::e4 * k4x[q]) +
-                     dp::e5 * k5x[q]) +
-                    dp::e6 * k6x[q];
-        double evv = ((((dp::e0 * k0v[q] + dp::e2 * k2v[q]) + dp::e3 * k3v[q]) +
-                       dp::e4 * k4v[q]) +
-                      dp::e5 * k5v[q]) +
-                     dp::e6 * k6v[q];
-        const int j = l * C + q;
-        double e1 = ex / (at(a, j) + rt(a, j) * fmax(fabs(x[q]), fabs(nx[q])));
-        double e2 = evv / (at(a, nm + j) + rt(a, nm + j) * fmax(fabs(v[q]), fabs(nv[q])));
-        err += e1 * e1 + e2 * e2;
-      }
+      const double ex = ((((dp::e0 * k0x[q] + dp::e2 * k2x[q]) + dp::e3 * k3x[q]) + dp::e4 * k4x[q]) + dp::e5 * k5x[q]) + dp::e6 * k6x[q];
+      const double ev2 = ((((dp::e0 * k0v[q] + dp::e2 * k2v[q]) + dp::e3 * k3v[q]) + dp::e4 * k4v[q]) + dp::e5 * k5v[q]) + dp::e6 * k6v[q];
+      // A mass beyond N takes mass 0's tolerances and adds nothing.
+      const bool real = l * C + q < nm;
+      const int j = real ? l * C + q : 0;
+      const double skx = at(a, j) + rt(a, j) * fmax(fabs(x[q]), fabs(nx[q]));
+      const double skv = at(a, nm + j) + rt(a, nm + j) * fmax(fabs(v[q]), fabs(nv[q]));
+      const double e1 = ex / skx, e2 = ev2 / skv;
+      const double e = e1 * e1 + e2 * e2;
+      en[q] = real ? e : 0.0;
     }
-    err = gsum(err);
+    double err = gsum(lane_sum(en));
     double deno = err;
     if (deno <= 0.0) deno = 1.0;
     err = fabs(h) * err * sqrt(1.0 / (deno * (double)(2 * nm)));
@@ -1822,18 +1896,17 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
     if (err <= 1.0) {
       double t_new = t + h;
       double dnx[C], dnv[C];
-      rhs(nx, nv, dnx, dnv);
+      rhs0(nx, nv, dnx, dnv);
       if (stiff_check) {
-        double stdnum = 0.0, stden = 0.0;
+        double ed[C];
 #pragma unroll
         for (int q = 0; q < C; ++q) {
           double u = segx[q] - k6x[q], u2 = segv[q] - k6v[q];
-          stdnum += u * u + u2 * u2;
+          en[q] = u * u + u2 * u2;
           double w = dnx[q] - sx[q], w2 = dnv[q] - sv[q];
-          stden += w * w + w2 * w2;
+          ed[q] = w * w + w2 * w2;
         }
-        stdnum = gsum(stdnum);
-        stden = gsum(stden);
+        const double stdnum = gsum(lane_sum(en)), stden = gsum(lane_sum(ed));
         if (stden > 0.0) {
           if (stiff_exceeds(h, stdnum, stden)) {
             nonstiff = 0;
@@ -1859,30 +1932,23 @@ struct GroupDopri5 : GroupCommon<G, C, OUT> {
         double c1x[C], c1v[C], c2x[C], c2v[C], c3x[C], c3v[C];
 #pragma unroll
         for (int q = 0; q < C; ++q) {
-          double dx = nx[q] + (-1.0) * x[q], dv2 = nv[q] + (-1.0) * v[q];
-          double bx = h * k0x[q] + (-1.0) * dx, bv = h * k0v[q] + (-1.0) * dv2;
+          const double dx = nx[q] - x[q], dv2 = nv[q] - v[q];
           c1x[q] = dx;
           c1v[q] = dv2;
-          c2x[q] = bx;
-          c2v[q] = bv;
-          c3x[q] = (dx + (-h) * dnx[q]) + (-1.0) * bx;
-          c3v[q] = (dv2 + (-h) * dnv[q]) + (-1.0) * bv;
+          c2x[q] = fma(h, k0x[q], -dx);
+          c2v[q] = fma(h, k0v[q], -dv2);
+          c3x[q] = fma(-h, dnx[q], dx) - c2x[q];
+          c3v[q] = fma(-h, dnv[q], dv2) - c2v[q];
         }
-        const double hp = h, tp = t, cont4 = 0.0 * h;
+        const double hp = h, tp = t;
         auto interp = [&](double te, double* ox, double* ov) {
           if (te < tp || te > t_new) return false;
-          double s = (te - tp) / hp;
-          double s1 = 1.0 - s;
+          const double s = (te - tp) / hp;
+          const double s1 = 1.0 - s;
 #pragma unroll
           for (int q = 0; q < C; ++q) {
-            double ax = cont4 * s1 + c3x[q];
-            ax = ax * s + c2x[q];
-            ax = ax * s1 + c1x[q];
-            ox[q] = x[q] + s * ax;
-            double av = cont4 * s1 + c3v[q];
-            av = av * s + c2v[q];
-            av = av * s1 + c1v[q];
-            ov[q] = v[q] + s * av;
+            ox[q] = fma(s, fma(fma(c3x[q], s, c2x[q]), s1, c1x[q]), x[q]);
+            ov[q] = fma(s, fma(fma(c3v[q], s, c2v[q]), s1, c1v[q]), v[q]);
           }
           return true;
         };

@@ -9,9 +9,9 @@
 //                 shape per size class (kernels_spring_group.hip).
 //   DE_MAP_AUTO   as DE_MAP_GROUP.  Systems are bucketed into size classes
 //                 (N <= 4, 8, ..., 256);
-//                 for each class of DOPRI5 an autotuner times every (G, C, block) with
-//                 G*C equal to the class cap on a sample of the class and keeps
-//                 the fastest.  Classes run concurrently on their own streams,
+//                 for each class of DOPRI5 an autotuner times the shapes (G, C)
+//                 with G*C equal to the class cap on a sample of the class and
+//                 keeps the fastest.  Classes run concurrently on their own streams,
 //                 each as a persistent kernel whose groups take the next system
 //                 of the class from a work counter when they finish one.
 #include <hip/hip_runtime.h>
@@ -77,7 +77,9 @@ spring_group_kernel(SpringArgs A) {
   spring_group_loop<GroupDopri5<G, C, OUT>>(A);
 }
 
-__global__ void spring_zero_counter(unsigned long long* c) { *c = 0ull; }
+__global__ void spring_zero_counters(unsigned long long* c, int n) {
+  if ((int)threadIdx.x < n) c[threadIdx.x] = 0ull;
+}
 
 struct Config {
   int g, c;
@@ -89,12 +91,76 @@ struct Config {
 static const Config kConfigs[] = {
     DE_CFG(4, 1),  DE_CFG(8, 1),  DE_CFG(16, 1), DE_CFG(32, 1), DE_CFG(64, 1),
     DE_CFG(2, 2),  DE_CFG(4, 2),  DE_CFG(8, 2),  DE_CFG(16, 2), DE_CFG(32, 2), DE_CFG(64, 2),
+    DE_CFG(8, 3),  DE_CFG(16, 3), DE_CFG(32, 3), DE_CFG(64, 3),
     DE_CFG(1, 4),  DE_CFG(2, 4),  DE_CFG(4, 4),  DE_CFG(8, 4),  DE_CFG(16, 4), DE_CFG(32, 4),
     DE_CFG(64, 4),
 };
 #undef DE_CFG
 static const int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
-static const int kBlocks[] = {64, 256};
+
+// The shapes the autotuner times: at least four lanes per system, and four masses
+// per lane only in the classes that need them.  (On the 64k-system ensemble, 2 000
+// to 10 000 systems per class: two lanes of two masses 0.73 against 0.63 ms for
+// four lanes of one; four masses per lane 0.79 to 1.28 against 0.65 to 0.98 ms up
+// to 64 masses, 1.16 against 1.22 ms at 128.)  Blocks of one wavefront leave their
+// slot as soon as its groups have drained.
+constexpr int kTunedBlock = 64;
+static bool tuned_shape(const Config& cf, int cap) {
+  return cf.g * cf.c == cap && cf.g >= 4 && (cf.c < 4 || cap >= 128);
+}
+
+// DOPRI5's size classes: the powers of two and, with three masses per lane, the
+// sizes between them: systems of log-uniform size then fill 85% of their lanes'
+// masses on average (72% with powers of two alone).
+static const int kDopri5Caps[] = {4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256};
+constexpr int kMaxClasses = sizeof(kDopri5Caps) / sizeof(kDopri5Caps[0]);
+static_assert(kNumCaps <= kMaxClasses, "per-class arrays");
+
+// The size classes of a method, and into which class each goes in one launch.
+// Every class is a kernel; those beyond the four hardware queues a process gets
+// wait for one another, and the longest solve bounds each.  So an ensemble whose
+// sizes span more than four classes uses only as many as it has systems for:
+//   few   64 lanes per system, one kernel per number of masses per lane;
+//   mid   (DOPRI5) five classes of 16 to 256 masses;
+//   all   every class.
+// A system keeps its sums' tree (three masses per lane or a power of two) in each
+// of them, so its result does not depend on the ensemble it is in.
+// Measured on chains of 4 to 256 masses, DOPRI5 at rtol 1e-6 over t in [0, 10],
+// few / mid / all in ms: 1024 systems 0.77 / - / 2.16, 4096 1.23 / 1.46 / 2.37,
+// 8192 1.92 / 1.83 / 2.75, 16384 3.44 / 2.62 / 3.44, 32768 6.44 / 4.67 / 4.67,
+// 65536 12.5 / 8.9 / 7.7; RK4 and DOP853, few / all: 1024 0.87 / 1.53 and 0.72 /
+// 1.20, 8192 1.75 / 2.09 and 1.75 / 2.31, 16384 3.19 / 3.14 and 3.16 / 3.23.
+constexpr int kQueues = 4;
+constexpr int64_t kFewSystems = 6144, kMidSystems = 32768;  // DOPRI5
+constexpr int64_t kFewSystemsMethod = 12288;                // the other methods
+enum Merge { kMergeAll = 0, kMergeMid = 1, kMergeFew = 2 };
+
+struct ClassSet {
+  const int* caps;
+  int n;
+};
+static ClassSet class_set(int method) {
+  return method == DE_METHOD_DOPRI5 ? ClassSet{kDopri5Caps, kMaxClasses}
+                                    : ClassSet{kCaps, kNumCaps};
+}
+static Merge merge_of(int method, int64_t systems, int classes) {
+  if (classes <= kQueues) return kMergeAll;
+  if (method != DE_METHOD_DOPRI5) return systems <= kFewSystemsMethod ? kMergeFew : kMergeAll;
+  return systems <= kFewSystems ? kMergeFew : (systems <= kMidSystems ? kMergeMid : kMergeAll);
+}
+// The class that `cap`'s systems are solved in.
+static int merged_cap(Merge m, int cap) {
+  const bool three = cap % 3 == 0;
+  if (m == kMergeFew) return three ? 192 : (cap <= 64 ? 64 : cap);
+  if (m == kMergeMid)
+    return three ? (cap <= 48 ? 48 : 192) : (cap <= 16 ? 16 : (cap <= 64 ? 64 : 256));
+  return cap;
+}
+static int class_index(const ClassSet& cs, int masses) {
+  int k = 0;
+  while (k < cs.n && cs.caps[k] < masses) ++k;
+  return k;
+}
 
 struct Choice {
   int cfg = -1;
@@ -109,17 +175,15 @@ struct Shape {
 
 // Process-wide state: autotune decisions per size class, streams, workspace.
 static std::mutex g_mu;
-static std::map<int, Choice> g_tuned;
-static hipStream_t g_streams[kNumCaps] = {};
-static hipEvent_t g_fork = nullptr, g_join[kNumCaps] = {};
+// DOPRI5's choices by class cap: the autotuner's, for ensembles that use every class
+// and for those that use five, and the caps solved with 64 lanes per system.
+// Which shape is picked does not change a system's result.
+static std::map<int, Choice> g_tuned[2];
+static std::map<int, Choice> g_few;
+static hipStream_t g_streams[kMaxClasses] = {};
+static hipEvent_t g_fork = nullptr, g_join[kMaxClasses] = {};
 static unsigned long long* g_counters = nullptr;
 static int g_num_cu = 0;
-
-static int cap_index(int nm) {
-  for (int k = 0; k < kNumCaps; ++k)
-    if (nm <= kCaps[k]) return k;
-  return -1;
-}
 
 static int ensure_runtime() {
   if (g_fork) return 0;
@@ -127,12 +191,12 @@ static int ensure_runtime() {
   if (hipGetDevice(&dev) != hipSuccess) return -1;
   if (hipDeviceGetAttribute(&g_num_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return -1;
-  for (int k = 0; k < kNumCaps; ++k) {
+  for (int k = 0; k < kMaxClasses; ++k) {
     if (hipStreamCreateWithFlags(&g_streams[k], hipStreamNonBlocking) != hipSuccess) return -1;
     if (hipEventCreateWithFlags(&g_join[k], hipEventDisableTiming) != hipSuccess) return -1;
   }
   if (hipEventCreateWithFlags(&g_fork, hipEventDisableTiming) != hipSuccess) return -1;
-  if (hipMalloc(&g_counters, sizeof(unsigned long long) * (kNumCaps + 1)) != hipSuccess) return -1;
+  if (hipMalloc(&g_counters, sizeof(unsigned long long) * (kMaxClasses + 1)) != hipSuccess) return -1;
   return 0;
 }
 
@@ -162,6 +226,7 @@ static const ClassKernel* method_kernels(int method) {
   return nullptr;
 }
 
+// The class's counter has been zeroed.
 static int launch_class(const SpringArgs& base, const int32_t* d_list, int64_t len,
                         int64_t work_share_blocks, const Shape& sh, unsigned long long* counter,
                         hipStream_t s) {
@@ -173,39 +238,54 @@ static int launch_class(const SpringArgs& base, const int32_t* d_list, int64_t l
   int64_t need = (len + groups_per_block - 1) / groups_per_block;
   int64_t grid = work_share_blocks < need ? work_share_blocks : need;
   if (grid < 1) grid = 1;
-  hipLaunchKernelGGL(spring_zero_counter, dim3(1), dim3(1), 0, s, counter);
   hipLaunchKernelGGL(sh.kernel, dim3((unsigned)grid), dim3(sh.block), 0, s, A);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Time every candidate for size class k on (up to) `sample` systems.
-static Choice autotune(const SpringArgs& base, int k, const int32_t* d_list, int64_t len,
+// The shape of 64 lanes for `cap` masses.
+static Choice wave_per_system(int cap) {
+  Choice ch;
+  ch.block = kTunedBlock;
+  for (int ci = 0; ci < kNumConfigs; ++ci)
+    if (kConfigs[ci].g == 64 && 64 * kConfigs[ci].c == cap) ch.cfg = ci;
+  return ch;
+}
+
+// Time every candidate for the size class of `cap` masses on (up to) 8192 systems.
+static Choice autotune(const SpringArgs& base, int cap, const int32_t* d_list, int64_t len,
                        hipStream_t s) {
   Choice best;
+  best.block = kTunedBlock;
+  int candidates = 0;
+  for (int ci = 0; ci < kNumConfigs; ++ci)
+    if (tuned_shape(kConfigs[ci], cap)) {
+      best.cfg = ci;
+      candidates += 1;
+    }
+  if (candidates <= 1) return best;
+  best.cfg = -1;
   float best_ms = 1e30f;
-  const int64_t sample = len < 1024 ? len : 1024;
+  const int64_t sample = len < 8192 ? len : 8192;
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return best;
   for (int ci = 0; ci < kNumConfigs; ++ci) {
-    if (kConfigs[ci].g * kConfigs[ci].c != kCaps[k]) continue;
-    for (int block : kBlocks) {
-      if (block < kConfigs[ci].g) continue;
-      Choice ch;
-      ch.cfg = ci;
-      ch.block = block;
-      int64_t full = (int64_t)g_num_cu * blocks_per_cu(class_kernel(base, kConfigs[ci]), block);
-      (void)hipEventRecord(e0, s);
-      if (launch_class(base, d_list, sample, full, shape_of(base, ch), g_counters + kNumCaps, s) !=
-          0)
-        continue;
-      (void)hipEventRecord(e1, s);
-      if (hipEventSynchronize(e1) != hipSuccess) continue;
-      float ms = 0.0f;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      if (ms < best_ms) {
-        best_ms = ms;
-        best = ch;
-      }
+    if (!tuned_shape(kConfigs[ci], cap)) continue;
+    Choice ch;
+    ch.cfg = ci;
+    ch.block = kTunedBlock;
+    const int64_t full =
+        (int64_t)g_num_cu * blocks_per_cu(class_kernel(base, kConfigs[ci]), ch.block);
+    unsigned long long* counter = g_counters + kMaxClasses;
+    (void)hipEventRecord(e0, s);
+    hipLaunchKernelGGL(spring_zero_counters, dim3(1), dim3(64), 0, s, counter, 1);
+    if (launch_class(base, d_list, sample, full, shape_of(base, ch), counter, s) != 0) continue;
+    (void)hipEventRecord(e1, s);
+    if (hipEventSynchronize(e1) != hipSuccess) continue;
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, e0, e1);
+    if (ms < best_ms) {
+      best_ms = ms;
+      best = ch;
     }
   }
   (void)hipEventDestroy(e0);
@@ -254,7 +334,7 @@ int64_t spring_workspace_bytes(const de_ode_batch* b) {
     return (int64_t)vectors * 512 * 8 * b->n +
            (b->points != DE_POINTS_NONE ? 8 * (b->n + 1) : 0);
   }
-  return (int64_t)sizeof(int32_t) * b->n + (int64_t)sizeof(unsigned long long) * (kNumCaps + 1) +
+  return (int64_t)sizeof(int32_t) * b->n + (int64_t)sizeof(unsigned long long) * (kMaxClasses + 1) +
          (b->points != DE_POINTS_NONE ? 8 * (b->n + 2) : 0);
 }
 
@@ -275,18 +355,21 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   base.list = nullptr;
   base.list_len = 0;
   // Host-side size scan: validity, total state length, classes.
+  const ClassSet cs = class_set(b->method);
   int64_t state_len = 0;
-  std::vector<std::vector<int32_t>> lists(kNumCaps);
-  std::vector<int64_t> masses(kNumCaps, 0);
+  std::vector<int64_t> count(cs.n, 0);
+  std::vector<uint8_t> class_of((size_t)n);
+  uint8_t class_of_size[257];
+  for (int m = 0; m <= 256; ++m) class_of_size[m] = (uint8_t)class_index(cs, m);
   const bool comp_event =
       b->event_solout != DE_SOLOUT_DEFAULT && a.ev.fn == kEventComponent;
   for (int64_t i = 0; i < n; ++i) {
-    int k = cap_index(host_sizes[i]);
-    if (host_sizes[i] < 1 || k < 0) return 1;
-    if (comp_event && b->event_component >= 2 * host_sizes[i]) return 3;
-    lists[k].push_back((int32_t)i);
-    masses[k] += host_sizes[i];
-    state_len += 2 * (int64_t)host_sizes[i];
+    const int32_t m = host_sizes[i];
+    if (m < 1 || m > 256) return 1;
+    if (comp_event && b->event_component >= 2 * m) return 3;
+    class_of[i] = class_of_size[m];
+    count[class_of[i]] += 1;
+    state_len += 2 * (int64_t)m;
   }
   const bool pts = b->points != DE_POINTS_NONE;
   std::vector<int64_t> ypos;
@@ -320,14 +403,26 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
     const hipError_t e = hipGetLastError();
     return hipFreeAsync(work, s) == hipSuccess && e == hipSuccess ? 0 : -1;
   }
-  // Group mapping: upload class lists (one buffer, classes back to back).
-  std::vector<int32_t> all;
-  std::vector<int64_t> start(kNumCaps + 1, 0);
-  for (int k = 0; k < kNumCaps; ++k) {
-    start[k] = (int64_t)all.size();
-    all.insert(all.end(), lists[k].begin(), lists[k].end());
+  // Group mapping: the launch's classes, and their lists to upload (one buffer,
+  // classes back to back).
+  const bool fixed_group = b->mapping == DE_MAP_GROUP && b->group_size > 0;
+  int classes = 0;
+  for (int k = 0; k < cs.n; ++k) classes += count[k] > 0 ? 1 : 0;
+  const Merge merge = fixed_group ? kMergeAll : merge_of(b->method, n, classes);
+  std::vector<int> merged(cs.n);
+  std::vector<int64_t> own = count;
+  count.assign(cs.n, 0);
+  for (int k = 0; k < cs.n; ++k) {
+    merged[k] = class_index(cs, merged_cap(merge, cs.caps[k]));
+    count[merged[k]] += own[k];
   }
-  start[kNumCaps] = (int64_t)all.size();
+  std::vector<int64_t> start(cs.n + 1, 0);
+  for (int k = 0; k < cs.n; ++k) start[k + 1] = start[k] + count[k];
+  std::vector<int32_t> all((size_t)n);
+  {
+    std::vector<int64_t> next(start.begin(), start.end() - 1);
+    for (int64_t i = 0; i < n; ++i) all[next[merged[class_of[i]]]++] = (int32_t)i;
+  }
   // The point states' offsets follow the lists, 8-byte aligned.
   const size_t list_bytes = (sizeof(int32_t) * (all.size() + 1) + 7) & ~(size_t)7;
   int32_t* d_list = nullptr;
@@ -345,41 +440,43 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   if (pts) base.pts_ypos = (const int64_t*)((const char*)d_list + list_bytes);
   // Choose a configuration per class.
   const ClassKernel* fixed = method_kernels(b->method);
-  std::vector<Shape> shape(kNumCaps);
-  for (int k = 0; k < kNumCaps; ++k) {
-    if (lists[k].empty()) continue;
+  std::vector<Shape> shape(cs.n);
+  for (int k = 0; k < cs.n; ++k) {
+    if (count[k] == 0) continue;
     if (fixed) {
       shape[k] = {fixed[k].k, fixed[k].g, kGroupBlock};
       continue;
     }
     Choice ch;
-    if (b->mapping == DE_MAP_GROUP && b->group_size > 0) {
+    if (fixed_group) {
       for (int ci = 0; ci < kNumConfigs; ++ci)
-        if (kConfigs[ci].g == b->group_size && kConfigs[ci].g * kConfigs[ci].c == kCaps[k])
+        if (kConfigs[ci].g == b->group_size && kConfigs[ci].g * kConfigs[ci].c == cs.caps[k])
           ch.cfg = ci;
       if (ch.cfg < 0) {
         // group size too small for this class: largest C that covers the cap
         for (int ci = 0; ci < kNumConfigs; ++ci)
-          if (kConfigs[ci].g * kConfigs[ci].c == kCaps[k] &&
+          if (kConfigs[ci].g * kConfigs[ci].c == cs.caps[k] &&
               (ch.cfg < 0 || kConfigs[ci].c > kConfigs[ch.cfg].c))
             ch.cfg = ci;
       }
     } else {
-      auto it = g_tuned.find(k);
-      if (it != g_tuned.end()) {
-        ch = it->second;
+      if (merge == kMergeFew) {
+        ch = wave_per_system(cs.caps[k]);
+        for (int o = 0; o < cs.n; ++o)
+          if (merged[o] == k && own[o] > 0) g_few[cs.caps[o]] = ch;
       } else {
-        ch = autotune(base, k, d_list + start[k], (int64_t)lists[k].size(), s);
-        if (ch.cfg < 0) {
-          (void)hipFreeAsync(d_list, s);
-          return -1;
-        }
-        g_tuned[k] = ch;
+        Choice& known = g_tuned[merge][cs.caps[k]];
+        if (known.cfg < 0) known = autotune(base, cs.caps[k], d_list + start[k], count[k], s);
+        ch = known;
+      }
+      if (ch.cfg < 0) {
+        (void)hipFreeAsync(d_list, s);
+        return -1;
       }
     }
     shape[k] = shape_of(base, ch);
   }
-  // Launch classes concurrently: the three small classes first, then the
+  // Launch classes concurrently: the three smallest classes first, then the
   // others largest first.  Every class kernel gets a full-device grid (capped
   // by its number of systems): the kernels are persistent and exit when their
   // class is drained, so blocks of the classes launched later are dispatched
@@ -387,21 +484,24 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   // The small classes (N <= 16) hold few waves whose long step sequences set
   // their time (latency, not throughput): started first, they run beside the
   // large classes instead of after them, and the largest class then starts
-  // next rather than running alone at the end (11.8 against 12.7 ms for the
-  // 64k-system ensemble, largest first).  (A fixed share per class left the
+  // next rather than running alone at the end (measured with seven classes:
+  // 11.8 against 12.7 ms for the 64k-system ensemble, largest first).  (A fixed share per class left the
   // GPU idle whenever classes waited behind others for one of the few
   // hardware queues a process gets; ordering each class's systems by size was
   // slower, 14.9 ms: it scatters the group's memory accesses.)
-  static const int kLaunchOrder[kNumCaps] = {0, 1, 2, 6, 5, 4, 3};
-  bool ok = hipEventRecord(g_fork, s) == hipSuccess;
-  for (int q = 0; q < kNumCaps && ok; ++q) {
-    const int k = kLaunchOrder[q];
-    if (lists[k].empty()) continue;
+  std::vector<int> launch_order;
+  for (int k = 0; k < cs.n && cs.caps[k] <= 16; ++k) launch_order.push_back(k);
+  for (int k = cs.n - 1; k >= 0 && cs.caps[k] > 16; --k) launch_order.push_back(k);
+  hipLaunchKernelGGL(spring_zero_counters, dim3(1), dim3(64), 0, s, g_counters, cs.n);
+  bool ok = hipGetLastError() == hipSuccess && hipEventRecord(g_fork, s) == hipSuccess;
+  for (int q = 0; q < cs.n && ok; ++q) {
+    const int k = launch_order[q];
+    if (count[k] == 0) continue;
     const Shape& sh = shape[k];
     int64_t share = (int64_t)g_num_cu * blocks_per_cu(sh.kernel, sh.block);
     ok = hipStreamWaitEvent(g_streams[k], g_fork, 0) == hipSuccess &&
-         launch_class(base, d_list + start[k], (int64_t)lists[k].size(), share, sh,
-                      g_counters + k, g_streams[k]) == 0 &&
+         launch_class(base, d_list + start[k], count[k], share, sh, g_counters + k,
+                      g_streams[k]) == 0 &&
          hipEventRecord(g_join[k], g_streams[k]) == hipSuccess &&
          hipStreamWaitEvent(s, g_join[k], 0) == hipSuccess;
   }
@@ -412,19 +512,26 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   return ok ? 0 : -1;
 }
 
-// Autotuner introspection: chosen (G, C, block) for size class cap, or -1.
+// Introspection: the shape (G, C, block) of the size class of `cap` masses, or -1
+// if none of its systems has been solved with a shape of the library's choice.
+// Where a class was only solved with 64 lanes per system, G is the number of those
+// that hold its masses.
 int spring_tuned(int cap, int* g, int* c, int* block) {
   std::lock_guard<std::mutex> lk(g_mu);
-  for (int k = 0; k < kNumCaps; ++k) {
-    if (kCaps[k] != cap) continue;
-    auto it = g_tuned.find(k);
-    if (it == g_tuned.end()) return -1;
+  for (const auto& tuned : g_tuned) {
+    auto it = tuned.find(cap);
+    if (it == tuned.end() || it->second.cfg < 0) continue;
     *g = kConfigs[it->second.cfg].g;
     *c = kConfigs[it->second.cfg].c;
     *block = it->second.block;
     return 0;
   }
-  return -1;
+  auto it = g_few.find(cap);
+  if (it == g_few.end()) return -1;
+  *c = kConfigs[it->second.cfg].c;
+  *g = cap / *c;
+  *block = it->second.block;
+  return 0;
 }
 
 }  // namespace parity

@@ -1,6 +1,6 @@
-"""GPU: the spring chains' group kernels of the methods beside DOPRI5 give the
-CPU restatement's values (as the one-lane mapping does), at the sizes where a
-size class or a lane's masses end."""
+"""GPU: the spring chains' group kernels at the sizes where a size class or a
+lane's masses end.  The methods beside DOPRI5 give the CPU restatement's values
+(as the one-lane mapping does); DOPRI5's shapes agree with one another."""
 import numpy as np
 import pytest
 
@@ -104,15 +104,67 @@ def test_values_that_overflow(orc, method):
     check(orc, ens, (DE_MAP_AUTO, DE_MAP_LANE))
 
 
-def test_results_do_not_depend_on_the_batch(orc):
-    # A system alone and among others gives the same bits.
-    sysm, y0 = chains([6, 40, 100, 200, 6, 40, 100, 200, 3], 75)
-    for method in ("dop853", "rkv656e", "rk4"):
-        whole = IVP.ode(sysm, 0.0, 2.0, y0).method(make(method)).solve()
-        for i in (2, 3, 8):
-            a, b = int(sysm.state_offset[i]), int(sysm.state_offset[i + 1])
-            pa, pb = int(sysm.param_offset[i]), int(sysm.param_offset[i + 1])
-            one = IVP.ode(SpringChain(sysm.sizes[i:i + 1], sysm.params_packed[pa:pb]), 0.0, 2.0,
-                          y0[a:b]).method(make(method)).solve()
-            assert np.array_equal(one.y, whole.y[a:b])
+@pytest.mark.parametrize("method,sizes", [("dopri5", (300, 6144, 6145, 32768, 32769)),
+                                          ("dop853", (300, 12288, 12289)),
+                                          ("rk4", (300, 12289))])
+def test_results_do_not_depend_on_the_batch(orc, method, sizes):
+    # The classes that a launch uses follow the number of systems; a system has
+    # the same bits alone, in a small ensemble and on either side of each rule.
+    edges = [6, 23, 40, 100, 160, 200, 3, 64]
+    rng = np.random.default_rng(75)
+    pool = np.concatenate([edges, rng.integers(1, 257, 92)])
+    sysm, y0 = chains(pool, 75)
+
+    def part(idx):
+        so, po = sysm.state_offset, sysm.param_offset
+        p = np.concatenate([sysm.params_packed[po[i]:po[i + 1]] for i in idx])
+        y = np.concatenate([y0[so[i]:so[i + 1]] for i in idx])
+        return IVP.ode(SpringChain(pool[idx], p), 0.0, 0.6, y).method(make(method, h=0.02))
+
+    alone = [part([i]).solve() for i in range(len(edges))]
+    if method != "dopri5":
+        assert all(np.array_equal(a.y, orc.solve_ode(part([i])).y) for i, a in enumerate(alone))
+    for n in sizes:
+        idx = np.concatenate([np.arange(len(edges)), rng.integers(0, len(pool), n - len(edges))])
+        whole = part(idx).solve()
+        for i, one in enumerate(alone):
+            assert np.array_equal(one.y, whole.final_state(i)), (n, i)
             assert one.accepted[0] == whole.accepted[i] and one.evals[0] == whole.evals[i]
+
+
+@pytest.mark.parametrize("out", ["final", "t_eval", "points", "event"])
+def test_dopri5_shapes_agree(orc, out):
+    # Every shape (lanes per system, masses per lane) of a size class adds the
+    # norm in one order, so the shape does not change a bit; against the oracle
+    # the sums' order and the fused interpolant leave roundings (the group
+    # mappings' bound: final state within 1e-10 of the state's largest value).
+    sysm, y0 = chains(EDGES, 76)
+    ens = IVP.ode(sysm, 0.0, 3.0, y0).method(make("dopri5"))
+    if out == "t_eval":
+        ens = ens.t_eval(np.linspace(-0.1, 3.0, 14))
+    elif out == "points":
+        ens = ens.even(0.21)
+    elif out == "event":
+        ens = ens.event(deamd.Event.component(0, 0.05))
+    want = orc.solve_ode(ens, threads=THREADS)
+    first = ens.options(mapping=DE_MAP_AUTO, group_size=0).solve()
+    for f in ("status", "accepted", "rejected", "evals"):
+        assert np.array_equal(getattr(first, f), getattr(want, f)), f
+    for i in range(len(EDGES)):
+        w = want.final_state(i)
+        assert np.abs(first.final_state(i) - w).max() <= 1e-10 * np.abs(w).max()
+    for g in (1, 2, 4, 8, 16, 32, 64):
+        got = ens.options(mapping=DE_MAP_GROUP, group_size=g).solve()
+        for f in ("status", "accepted", "rejected", "evals", "t", "y", "dense", "n_dense",
+                  "n_events", "n_points"):
+            a, b = getattr(got, f), getattr(first, f)
+            assert (a is None) == (b is None)
+            if a is not None:
+                assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f"), (f, g)
+        if out == "points":
+            for i in range(len(EDGES)):
+                for a, b in zip(got.points(i), first.points(i)):
+                    assert np.array_equal(a, b)
+        if out == "event":
+            assert np.array_equal(got.event_t, first.event_t, equal_nan=True)
+            assert np.array_equal(got.event_y, first.event_y, equal_nan=True)
