@@ -73,11 +73,12 @@ DE_HD double as_f64(uint64_t u) {
 DE_HD double signum(double x) { return x != x ? x : copysign(1.0, x); }
 
 // constrain_step_size (src/utils.rs:22-33): clamp |h| to [h_min, h_max] keeping
-// the sign of h (written with selects; a NaN h is returned unchanged).
+// the sign of h (written with selects; a NaN h is returned unchanged).  signum(h)
+// times a bound is the bound with its sign flipped where h's is set.
 DE_HD double constrain_step_size(double h, double h_min, double h_max) {
-  const double sign = signum(h);
+  const uint64_t sign = as_u64(h) & 0x8000000000000000ULL;
   const double a = fabs(h);
-  return a < h_min ? sign * h_min : (a > h_max ? sign * h_max : h);
+  return a < h_min ? as_f64(as_u64(h_min) ^ sign) : (a > h_max ? as_f64(as_u64(h_max) ^ sign) : h);
 }
 
 // The stiffness test's decision h * sqrt(num / den) > 6.1, with den > 0, as

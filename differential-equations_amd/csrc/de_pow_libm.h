@@ -89,10 +89,10 @@ DE_HD double uflow(uint64_t sign) { return sign ? -0.0 : 0.0; }
 // subnormal) x.
 DE_HD DE_FORCE_INLINE double log_inline(uint64_t ix, double* tail) {
   DE_NO_CONTRACT
-  const uint64_t tmp = ix - kOff;
-  // Integer steps on the high word (the low one of tmp & 0xfff << 52 is 0):
+  // Integer steps on the high words (the low word of kOff is 0): tmp = ix - kOff,
   // i = bits 45..51 of tmp, k = its top 12 bits signed, z = x / 2^k.
-  const uint32_t thi = (uint32_t)(tmp >> 32);
+  static_assert((uint32_t)kOff == 0, "tmp's high word takes no borrow");
+  const uint32_t thi = (uint32_t)(ix >> 32) - (uint32_t)(kOff >> 32);
   const int i = (int)((thi >> 13) & 127u);
   const int32_t k = (int32_t)thi >> 20;
   const uint32_t zhi = (uint32_t)(ix >> 32) - (thi & 0xfff00000u);
@@ -225,6 +225,51 @@ DE_HD double libm_pow(double x, double y) {
   const double ehi = y * hi;
   const double elo = fma(y, lo, fma(y, hi, -ehi));
   return exp_inline(ehi, elo, sign_bias);
+}
+
+// libm_pow(x, y) for a constant y with 2^-10 <= |y| < 1/2, as the controllers'
+// and the initial step's -1/order and 1/order, in fewer operations.  What such an
+// exponent rules out:
+//   y is no integer, so a negative x (but -0 and -inf) gives NaN and no sign is kept;
+//   |y log x| <= 1074 ln 2 / 2 < 512: no overflow, underflow or rescaled result;
+//   |y log x| < 2^-54, where libm_pow returns 1 + y log x: that sum and the general
+//   expression both round to 1.
+// tests/test_pow_const.py holds it to libm_pow's bits.  62 vector instructions
+// against 88: 1 M Lorenz trajectories with DOPRI5 over t in [0, 50] take 60.7
+// against 62.2 ms, 1024 over [0, 20] 4.32 against 4.47 ms.
+DE_HD DE_FORCE_INLINE double libm_pow_const(double x, double y) {
+  DE_NO_CONTRACT
+  using namespace libm_pow_detail;
+  uint64_t ix = as_u64(x);
+  if ((uint32_t)(ix >> 32) - 0x00100000u >= 0x7fe00000u) {
+    // x subnormal, zero, negative, inf or NaN.
+    if (zeroinfnan(ix)) {
+      const double x2 = x * x;
+      return y < 0.0 ? 1.0 / x2 : x2;
+    }
+    if (ix >> 63) return (x - x) / (x - x);
+    ix = as_u64(x * 0x1p52) - (52ULL << 52);
+  }
+  double lo;
+  const double hi = log_inline(ix, &lo);
+  const double ehi = y * hi;
+  const double elo = fma(y, lo, fma(y, hi, -ehi));
+  // exp(ehi + elo), as exp_inline's general path; 2^(ki / 128)'s bits differ from
+  // its table entry's in the high word only.
+  const double kd0 = fma(ehi, kInvLn2N, kShift);
+  const uint32_t ki = (uint32_t)as_u64(kd0);
+  const double kd = kd0 - kShift;
+  double r = fma(kd, kNegLn2loN, fma(kd, kNegLn2hiN, ehi));
+  r = elo + r;
+  const uint32_t idx = 2 * (ki & 127u);
+  const double tail = as_f64(kLibmPowExp[idx]);
+  const uint64_t base = kLibmPowExp[idx + 1];
+  const uint32_t top = (uint32_t)(base >> 32) + (ki << 13);
+  const double scale = as_f64(((uint64_t)top << 32) | (uint32_t)base);
+  const double r2 = r * r;
+  const double t = fma(r2, fma(r, kC3, kC2), r + tail);
+  const double tmp = fma(r2 * r2, fma(r, kC5, kC4), t);
+  return fma(tmp, scale, scale);
 }
 
 }  // namespace de

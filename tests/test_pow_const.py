@@ -1,0 +1,37 @@
+"""The controllers' pow (csrc/de_pow_libm.h, libm_pow_const) on the host: the bits
+of libm_pow for every exponent in use, over all regimes of x -- random bit
+patterns (negative, subnormal, NaN), error norms, arguments near 1 (where y log x
+falls below 2^-54), the table's interval ends and the special values."""
+import os
+import subprocess
+
+import numpy as np
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+EXE = os.path.join(HERE, "cpp", "_build", "pow_check")
+
+
+def arguments():
+    rng = np.random.default_rng(7)
+    bits = rng.integers(0, 2 ** 64, 200000, dtype=np.uint64).view(np.float64)
+    norms = 10.0 ** rng.uniform(-300, 300, 200000)
+    usual = 10.0 ** rng.uniform(-12, 4, 200000)
+    k = rng.integers(-(1 << 14), 1 << 14, 100000)
+    near = np.concatenate([1.0 + k * 2.0 ** -52, 1.0 + k * 2.0 ** -53])
+    sub = rng.integers(1, 1 << 52, 50000, dtype=np.uint64).view(np.float64)
+    edges = (np.uint64(0x3fe6955500000000) + (np.arange(0, 129, dtype=np.uint64) << np.uint64(45)))
+    ends = np.concatenate([(edges + np.uint64(d)).view(np.float64) for d in (0, 1)] +
+                          [(edges - np.uint64(1)).view(np.float64)])
+    scaled = np.concatenate([ends * 2.0 ** e for e in (-1021, -900, -60, -1, 1, 52, 700, 1022)])
+    special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, -np.nan, 1.0, -1.0, 5e-324, -5e-324,
+                        2.2250738585072014e-308, 2.225073858507201e-308, 1.7976931348623157e308])
+    with np.errstate(all="ignore"):
+        return np.concatenate([bits, norms, usual, near, sub, ends, scaled, special])
+
+
+def test_pow_const_has_libm_pow_bits():
+    if not os.path.exists(EXE):
+        subprocess.check_call(["make", "-s", "-C", os.path.join(HERE, "cpp"), "_build/pow_check"])
+    out = subprocess.run([EXE], input=arguments().tobytes(), capture_output=True, timeout=300)
+    assert out.returncode == 0, out.stdout.decode()[-2000:]
+    assert b", 0 differ" in out.stdout
