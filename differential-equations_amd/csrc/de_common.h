@@ -72,6 +72,22 @@ DE_HD double as_f64(uint64_t u) {
 // values, NaN for NaN.
 DE_HD double signum(double x) { return x != x ? x : copysign(1.0, x); }
 
+// A pointer known to hold global memory, as such.  The lanes' kernels read their
+// pointers from an argument block in memory, where the compiler only knows generic
+// ones: their accesses would be flat, which count among the scalar loads' waits, so
+// that the next attempt's settings would wait for the last output's store.
+#if defined(__HIP_DEVICE_COMPILE__)
+template <class T>
+DE_DEV __attribute__((address_space(1))) T* global_ptr(T* p) {
+  return (__attribute__((address_space(1))) T*)p;
+}
+#else
+template <class T>
+DE_HD T* global_ptr(T* p) {
+  return p;
+}
+#endif
+
 // constrain_step_size (src/utils.rs:22-33): clamp |h| to [h_min, h_max] keeping
 // the sign of h (written with selects; a NaN h is returned unchanged).  signum(h)
 // times a bound is the bound with its sign flipped where h's is set.

@@ -100,16 +100,16 @@ struct ErkLane {
       }
     }
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.y_final[c * a.n + i] = L.y[c];
-    a.t_final[i] = L.t;
-    a.accepted[i] = L.acc;
-    a.rejected[i] = L.rej;
-    a.evals[i] = st == kBadInput ? 0
+    for (int c = 0; c < D; ++c) global_ptr(a.y_final)[c * a.n + i] = L.y[c];
+    global_ptr(a.t_final)[i] = L.t;
+    global_ptr(a.accepted)[i] = L.acc;
+    global_ptr(a.rejected)[i] = L.rej;
+    global_ptr(a.evals)[i] = st == kBadInput ? 0
                                  : (int64_t)L.base_ev + (int64_t)(S - 1) * (L.acc + L.rej) +
                                        (int64_t)kAccEvals * L.acc;
-    a.status[i] = st;
-    if (DENSE && a.n_dense) a.n_dense[i] = L.pushed;
-    if (DENSE && EV == 0 && a.n_pts) a.n_pts[i] = L.pushed;
+    global_ptr(a.status)[i] = st;
+    if (DENSE && a.n_dense) global_ptr(a.n_dense)[i] = L.pushed;
+    if (DENSE && EV == 0 && a.n_pts) global_ptr(a.n_pts)[i] = L.pushed;
     if (DENSE && a.n_eval > 0) teval_tail_nan<D>(a, i, L.next_eval);
     if constexpr (EV != 0) {
       if (a.ev.brk)
@@ -128,10 +128,10 @@ struct ErkLane {
   DE_HD static void entry_root(const OdeArgs& a, int64_t i, const double* ent, double* res) {
     double meta[kEntryMeta];
 #pragma unroll
-    for (int m = 0; m < kEntryMeta; ++m) meta[m] = ent[m];
+    for (int m = 0; m < kEntryMeta; ++m) meta[m] = global_ptr(ent)[m];
     const double tp = meta[kEntryT0], hp = meta[kEntryH];
     const double t_new = tp + hp;
-    const double* d = ent + kEntryMeta;
+    const auto* d = global_ptr(ent) + kEntryMeta;
     if constexpr (kBi) {
       double yp[D], k[I][D];
       uint32_t bad[D];
@@ -188,13 +188,13 @@ struct ErkLane {
   DE_HD static double predicted_cost(const OdeArgs& a, int64_t i) {
     F f;
     f.load(a.params, a.n, i);
-    const double t0 = a.t0 ? a.t0[i] : a.t0s;
-    const double tf = a.tf ? a.tf[i] : a.tfs;
+    const double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    const double tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     double h0 = a.h0;
     if (h0 == 0.0 && tf != t0) {
       double y[D];
 #pragma unroll
-      for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+      for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
       LaneTol<D, VTOL> tl;
       tl.load(a, i);
       h0 = lane_h_init<F, LaneTol<D, VTOL>, O>(f, t0, tf, y, tl, a.h_min, a.h_max);
@@ -206,11 +206,11 @@ struct ErkLane {
   // evaluations plus two more, then f(t0, y0).
   DE_HD bool init(const OdeArgs& a, int64_t i) {
     f.load(a.params, a.n, i);
-    double t0 = a.t0 ? a.t0[i] : a.t0s;
-    tf = a.tf ? a.tf[i] : a.tfs;
+    double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     tol.load(a, i);
 #pragma unroll
-    for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+    for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
     t = t0;
     acc = rej = 0;
     pushed = 0;
@@ -462,7 +462,7 @@ struct ErkLane {
       const bool teval_out = DENSE && EV != 2 && a.n_eval > 0;
       bool tev = false;
       if (teval_out && accept && next_eval < a.n_eval) {
-        const double te = a.t_eval[next_eval];
+        const double te = global_ptr(a.t_eval)[next_eval];
         tev = !(dir > 0.0 ? te > t_new : te < t_new);
       }
       // Without a t_eval output the Solution's last point is the step's end
@@ -510,7 +510,7 @@ struct ErkLane {
               bool overflow = false;
               double* ent = ev.defer(a.ev, i, true, tp, hp, tail, pushed, &overflow);
               if (ent) {
-                double* dst = ent + kEntryMeta;
+                auto* dst = global_ptr(ent) + kEntryMeta;
                 if constexpr (kBi) {
 #pragma unroll
                   for (int c = 0; c < D; ++c) dst[c] = y[c];

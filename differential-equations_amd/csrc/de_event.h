@@ -94,7 +94,7 @@ DE_HD double event_g(const EventArgs& e, double value, double t, const double* y
   }
   double s = 0.0;
 #pragma unroll
-  for (int c = 0; c < D; ++c) s = s + (y[c] + (-1.0) * e.point[c]) * e.normal[c];
+  for (int c = 0; c < D; ++c) s = s + (y[c] + (-1.0) * global_ptr(e.point)[c]) * global_ptr(e.normal)[c];
   return s;
 }
 
@@ -102,23 +102,22 @@ DE_HD double event_g(const EventArgs& e, double value, double t, const double* y
 DE_HD bool sign_differs(double a, double b) { return !(signum(a) == signum(b)); }
 
 // Writes point k of trajectory i when it fits.
-template <int D>
-DE_HD void event_store(const EventArgs& e, int64_t n, int64_t i, int32_t k, double t,
-                       const double* y) {
+template <int D, class Y>
+DE_HD void event_store(const EventArgs& e, int64_t n, int64_t i, int32_t k, double t, Y y) {
   if (k < e.max_events) {
-    e.t_out[(int64_t)k * n + i] = t;
+    global_ptr(e.t_out)[(int64_t)k * n + i] = t;
 #pragma unroll
-    for (int c = 0; c < D; ++c) e.y_out[((int64_t)k * D + c) * n + i] = y[c];
+    for (int c = 0; c < D; ++c) global_ptr(e.y_out)[((int64_t)k * D + c) * n + i] = y[c];
   }
 }
 
 // Count and NaN for the slots past the last point.
 template <int D>
 DE_HD void event_finish(const EventArgs& e, int64_t n, int64_t i, int32_t pushed) {
-  if (e.n_out) e.n_out[i] = pushed;
+  if (e.n_out) global_ptr(e.n_out)[i] = pushed;
   for (int32_t k = pushed; k < e.max_events; ++k) {
-    e.t_out[(int64_t)k * n + i] = as_f64(kNaNBits);
-    for (int c = 0; c < D; ++c) e.y_out[((int64_t)k * D + c) * n + i] = as_f64(kNaNBits);
+    global_ptr(e.t_out)[(int64_t)k * n + i] = as_f64(kNaNBits);
+    for (int c = 0; c < D; ++c) global_ptr(e.y_out)[((int64_t)k * D + c) * n + i] = as_f64(kNaNBits);
   }
 }
 
@@ -225,7 +224,8 @@ DE_HD double* event_defer(const EventArgs& e, int64_t i, int32_t& k, bool need, 
     *overflow = true;
     return nullptr;
   }
-  double* ent = e.brk + ((i - e.base) * e.bmax + k) * e.width;
+  double* entry = e.brk + ((i - e.base) * e.bmax + k) * e.width;
+  auto* ent = global_ptr(entry);
   ent[kEntryT0] = t0;
   ent[kEntryH] = h;
   ent[kEntryG0] = g0;
@@ -233,14 +233,15 @@ DE_HD double* event_defer(const EventArgs& e, int64_t i, int32_t& k, bool need, 
   ent[kEntryTail] = tail;
   ent[kEntryTevals] = (double)tevals;
   k += 1;
-  return ent;
+  return entry;
 }
 
 // Result record of a root search.
 template <int D>
-DE_HD void event_result(double* r, int flag, double t, const double* y, double tail,
+DE_HD void event_result(double* record, int flag, double t, const double* y, double tail,
                         double tevals) {
   static_assert(4 + D <= kResWidth, "result record");
+  auto* r = global_ptr(record);
   r[kResFlag] = (double)flag;
   r[kResT] = t;
 #pragma unroll
@@ -252,7 +253,7 @@ DE_HD void event_result(double* r, int flag, double t, const double* y, double t
 // Deferred-mode end of a trajectory: the bracket count (the bookkeeping pass
 // writes the event outputs), or -1 after an overflow.
 DE_HD void event_defer_finish(const EventArgs& e, int64_t i, int32_t k, bool overflow) {
-  e.bcount[i - e.base] = overflow ? -1 : k;
+  global_ptr(e.bcount)[i - e.base] = overflow ? -1 : k;
 }
 
 // EventWrappedSolout around DefaultSolout or TEvalSolout.
@@ -268,7 +269,7 @@ struct LaneEvent<D, 1> {
   }
   // The solout call after init: only records g(t0, y0) (event.rs:346-355).
   DE_HD void start(const EventArgs& e, int64_t i, double t0, const double* y0) {
-    value = e.value_traj ? e.value_traj[i] : e.value;
+    value = e.value_traj ? global_ptr(e.value_traj)[i] : e.value;
     last_g = event_g<D>(e, value, t0, y0);
     count = 0;
   }
@@ -339,7 +340,7 @@ struct LaneEvent<D, 1> {
   DE_HD static void root(const EventArgs& e, int64_t i, const double* ent, double* res,
                          double t_prev, double t_curr, double dir, bool teval_base,
                          Interp& interp) {
-    const double v = e.value_traj ? e.value_traj[i] : e.value;
+    const double v = e.value_traj ? global_ptr(e.value_traj)[i] : e.value;
     double a = t_prev, b = t_curr, fa = ent[kEntryG0], fb = ent[kEntryG1];
     if ((dir > 0.0 && a > b) || (dir < 0.0 && a < b)) {
       double x = a;
@@ -366,13 +367,13 @@ struct LaneEvent<D, 1> {
   // (a reference panic) sends the trajectory to the inline solve, which
   // rewrites all of its outputs.
   DE_HD static bool book(const EventArgs& e, int64_t n, int64_t i, bool teval_base) {
-    const int32_t cnt = e.bcount[i - e.base];
+    const int32_t cnt = global_ptr(e.bcount)[i - e.base];
     if (cnt < 0) return false;
-    const double* base = e.res + (i - e.base) * e.bmax * kResWidth;
+    const auto* base = global_ptr(e.res) + (i - e.base) * e.bmax * kResWidth;
     int32_t pushed = 0;
     double tail = as_f64(kNaNBits), tevals = 0.0;
     for (int32_t k = 0; k < cnt; ++k) {
-      const double* r = base + (int64_t)k * kResWidth;
+      const auto* r = base + (int64_t)k * kResWidth;
       const double flag = r[kResFlag];
       if (flag == (double)kResPanic) return false;
       if (teval_base && r[kResY + D + 1] != tevals) {
@@ -407,7 +408,7 @@ struct LaneEvent<D, 2> {
     k = 0;
   }
   DE_HD void start(const EventArgs& e, int64_t i, double t0, const double* y0) {
-    value = e.value_traj ? e.value_traj[i] : e.value;
+    value = e.value_traj ? global_ptr(e.value_traj)[i] : e.value;
     last = event_g<D>(e, value, t0, y0);
   }
   DE_HD bool pre(const EventArgs& e, double t_curr, const double* y_curr) {
@@ -499,7 +500,7 @@ struct LaneEvent<D, 2> {
   DE_HD static void root(const EventArgs& e, int64_t i, const double* ent, double* res,
                          double t_prev, double t_curr, double, bool, Interp& interp) {
     LaneEvent<D, 2> s;
-    s.value = e.value_traj ? e.value_traj[i] : e.value;
+    s.value = e.value_traj ? global_ptr(e.value_traj)[i] : e.value;
     const double lo = ent[kEntryG0], off = ent[kEntryG1];
     bool found = false;
     double tc = 0.0, yc[D];
@@ -514,12 +515,12 @@ struct LaneEvent<D, 2> {
     event_result<D>(res, flag, tc, yc, 0.0, 0.0);
   }
   DE_HD static bool book(const EventArgs& e, int64_t n, int64_t i, bool) {
-    const int32_t cnt = e.bcount[i - e.base];
+    const int32_t cnt = global_ptr(e.bcount)[i - e.base];
     if (cnt < 0) return false;
-    const double* base = e.res + (i - e.base) * e.bmax * kResWidth;
+    const auto* base = global_ptr(e.res) + (i - e.base) * e.bmax * kResWidth;
     int32_t pushed = 0;
     for (int32_t k = 0; k < cnt; ++k) {
-      const double* r = base + (int64_t)k * kResWidth;
+      const auto* r = base + (int64_t)k * kResWidth;
       if (r[kResFlag] == (double)kResPanic) return false;
       event_store<D>(e, n, i, pushed, r[kResT], r + kResY);
       pushed += 1;

@@ -41,9 +41,9 @@ struct LorenzRhs {
   static constexpr int kParams = 3;
   double sigma, rho, beta;
   DE_HD void load(const double* p, int64_t stride, int64_t i) {
-    sigma = p[i];
-    rho = p[stride + i];
-    beta = p[2 * stride + i];
+    sigma = global_ptr(p)[i];
+    rho = global_ptr(p)[stride + i];
+    beta = global_ptr(p)[2 * stride + i];
   }
   DE_HD void diff(double, const double* y, double* dydt) const {
     double x = y[0], yv = y[1], z = y[2];
@@ -59,7 +59,7 @@ struct VanDerPolRhs {
   static constexpr int kDim = 2;
   static constexpr int kParams = 1;
   double mu;
-  DE_HD void load(const double* p, int64_t, int64_t i) { mu = p[i]; }
+  DE_HD void load(const double* p, int64_t, int64_t i) { mu = global_ptr(p)[i]; }
   DE_HD void diff(double, const double* y, double* dydt) const {
     double y1 = y[0], y2 = y[1];
     dydt[0] = y2;
@@ -73,7 +73,7 @@ struct ExponentialRhs {
   static constexpr int kDim = 1;
   static constexpr int kParams = 1;
   double k;
-  DE_HD void load(const double* p, int64_t, int64_t i) { k = p[i]; }
+  DE_HD void load(const double* p, int64_t, int64_t i) { k = global_ptr(p)[i]; }
   DE_HD void diff(double, const double* y, double* dydt) const {
     dydt[0] = k * y[0];
   }
@@ -86,8 +86,8 @@ struct LinearRhs {
   static constexpr int kParams = 2;
   double a, b;
   DE_HD void load(const double* p, int64_t stride, int64_t i) {
-    a = p[i];
-    b = p[stride + i];
+    a = global_ptr(p)[i];
+    b = global_ptr(p)[stride + i];
   }
   DE_HD void diff(double, const double* y, double* dydt) const {
     dydt[0] = a + b * y[0];
@@ -100,7 +100,7 @@ struct HarmonicRhs {
   static constexpr int kDim = 2;
   static constexpr int kParams = 1;
   double k;
-  DE_HD void load(const double* p, int64_t, int64_t i) { k = p[i]; }
+  DE_HD void load(const double* p, int64_t, int64_t i) { k = global_ptr(p)[i]; }
   DE_HD void diff(double, const double* y, double* dydt) const {
     dydt[0] = y[1];
     dydt[1] = -k * y[0];
@@ -114,8 +114,8 @@ struct LogisticRhs {
   static constexpr int kParams = 2;
   double k, m;
   DE_HD void load(const double* p, int64_t stride, int64_t i) {
-    k = p[i];
-    m = p[stride + i];
+    k = global_ptr(p)[i];
+    m = global_ptr(p)[stride + i];
   }
   DE_HD void diff(double, const double* y, double* dydt) const {
     dydt[0] = k * y[0] * (1.0 - y[0] / m);
@@ -172,9 +172,9 @@ struct OrnsteinUhlenbeckSde {
   double theta[D], mu[D], sigma[D];
   DE_HD void load(const double* p, int64_t stride, int64_t i) {
     for (int c = 0; c < D; ++c) {
-      theta[c] = p[(3 * c + 0) * stride + i];
-      mu[c] = p[(3 * c + 1) * stride + i];
-      sigma[c] = p[(3 * c + 2) * stride + i];
+      theta[c] = global_ptr(p)[(3 * c + 0) * stride + i];
+      mu[c] = global_ptr(p)[(3 * c + 1) * stride + i];
+      sigma[c] = global_ptr(p)[(3 * c + 2) * stride + i];
     }
   }
   DE_HD void drift(double, const double* y, double* f) const {
@@ -197,8 +197,8 @@ struct LinearDiagonalSde {
   double a[D], b[D];
   DE_HD void load(const double* p, int64_t stride, int64_t i) {
     for (int c = 0; c < D; ++c) {
-      a[c] = p[(2 * c + 0) * stride + i];
-      b[c] = p[(2 * c + 1) * stride + i];
+      a[c] = global_ptr(p)[(2 * c + 0) * stride + i];
+      b[c] = global_ptr(p)[(2 * c + 1) * stride + i];
     }
   }
   DE_HD void drift(double, const double* y, double* f) const {

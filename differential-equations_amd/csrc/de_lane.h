@@ -85,8 +85,8 @@ template <int D, bool V>
 struct LaneTol {
   double r, a;
   DE_HD void load(const OdeArgs& A, int64_t i) {
-    r = A.rtol_traj ? A.rtol_traj[i] : A.rtol;
-    a = A.atol_traj ? A.atol_traj[i] : A.atol;
+    r = A.rtol_traj ? global_ptr(A.rtol_traj)[i] : A.rtol;
+    a = A.atol_traj ? global_ptr(A.atol_traj)[i] : A.atol;
   }
   DE_HD double rt(int) const { return r; }
   DE_HD double at(int) const { return a; }
@@ -95,12 +95,12 @@ template <int D>
 struct LaneTol<D, true> {
   double r[D], a[D];
   DE_HD void load(const OdeArgs& A, int64_t i) {
-    const double rs = A.rtol_traj ? A.rtol_traj[i] : A.rtol;
-    const double as = A.atol_traj ? A.atol_traj[i] : A.atol;
+    const double rs = A.rtol_traj ? global_ptr(A.rtol_traj)[i] : A.rtol;
+    const double as = A.atol_traj ? global_ptr(A.atol_traj)[i] : A.atol;
 #pragma unroll
     for (int c = 0; c < D; ++c) {
-      r[c] = A.rtol_comp ? A.rtol_comp[c * A.n + i] : rs;
-      a[c] = A.atol_comp ? A.atol_comp[c * A.n + i] : as;
+      r[c] = A.rtol_comp ? global_ptr(A.rtol_comp)[c * A.n + i] : rs;
+      a[c] = A.atol_comp ? global_ptr(A.atol_comp)[c * A.n + i] : as;
     }
   }
   DE_HD double rt(int c) const { return r[c]; }
@@ -152,7 +152,7 @@ DE_HD bool teval_emit(const OdeArgs& a, int64_t i, double dir, int32_t& next, in
   int32_t idx = next;
   bool ok = true;
   while (idx < a.n_eval) {
-    double te = a.t_eval[idx];
+    double te = global_ptr(a.t_eval)[idx];
     bool in_range = dir > 0.0 ? ((te == t_prev && idx == 0) || (te > t_prev && te <= t_curr))
                               : ((te == t_prev && idx == 0) || (te < t_prev && te >= t_curr));
     if (in_range) {
@@ -165,14 +165,14 @@ DE_HD bool teval_emit(const OdeArgs& a, int64_t i, double dir, int32_t& next, in
         break;
       }
 #pragma unroll
-      for (int c = 0; c < D; ++c) a.dense[((int64_t)idx * D + c) * a.n + i] = out[c];
+      for (int c = 0; c < D; ++c) global_ptr(a.dense)[((int64_t)idx * D + c) * a.n + i] = out[c];
       pushed += 1;
       tail = te;
       idx += 1;
     } else {
       if ((dir > 0.0 && te > t_curr) || (dir < 0.0 && te < t_curr)) break;
 #pragma unroll
-      for (int c = 0; c < D; ++c) a.dense[((int64_t)idx * D + c) * a.n + i] = as_f64(kNaNBits);
+      for (int c = 0; c < D; ++c) global_ptr(a.dense)[((int64_t)idx * D + c) * a.n + i] = as_f64(kNaNBits);
       idx += 1;
     }
   }
@@ -184,7 +184,7 @@ template <int D>
 DE_HD void teval_tail_nan(const OdeArgs& a, int64_t i, int32_t from) {
   for (int32_t e = from; e < a.n_eval; ++e)
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.dense[((int64_t)e * D + c) * a.n + i] = as_f64(kNaNBits);
+    for (int c = 0; c < D; ++c) global_ptr(a.dense)[((int64_t)e * D + c) * a.n + i] = as_f64(kNaNBits);
 }
 
 // Variable-count point outputs: DefaultSolout (src/solout/default.rs:71-91),
@@ -197,11 +197,11 @@ enum : int32_t { kPointsNone = 0, kPointsSteps = 1, kPointsDense = 2, kPointsEve
 
 template <int D>
 DE_HD void points_push(const OdeArgs& a, int64_t i, int32_t& pushed, double t, const double* y) {
-  const int64_t s = a.pts_offset[i] + pushed;
-  if (s < a.pts_offset[i + 1]) {
-    a.pts_t[s] = t;
+  const int64_t s = global_ptr(a.pts_offset)[i] + pushed;
+  if (s < global_ptr(a.pts_offset)[i + 1]) {
+    global_ptr(a.pts_t)[s] = t;
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.pts_y[s * D + c] = y[c];
+    for (int c = 0; c < D; ++c) global_ptr(a.pts_y)[s * D + c] = y[c];
   }
   pushed += 1;
 }
@@ -314,9 +314,11 @@ struct Dopri5Lane {
   static constexpr int kEv = EV;
   static constexpr int kWavesPerEu = 3;  // occupancy hint of the persistent kernel
   static constexpr bool kLiveStep = true;  // step(a, i, live_in): lanes without work ride along
-  // Deferred event bracket: the meta fields, then y, y_new, f(t, y) and
-  // f(t_new, y_new); the root pass forms the interpolant from them.
-  static constexpr int kEntryWidth = kEntryMeta + 4 * D;
+  // Deferred event bracket: the meta fields, then y and y_new; the root pass
+  // evaluates f at both ends again (the same inputs and operations, so the same
+  // bits) and forms the interpolant.  Some lane of a wavefront brackets in nearly
+  // every attempt, so each value stored is a store instruction per attempt.
+  static constexpr int kEntryWidth = kEntryMeta + 2 * D;
   F f;
   double y[D], k0[D];
   double t, h, h_prev, tf, dir;
@@ -337,15 +339,15 @@ struct Dopri5Lane {
       }
     }
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.y_final[c * a.n + i] = L.y[c];
-    a.t_final[i] = L.t;
-    a.accepted[i] = L.acc;
-    a.rejected[i] = L.rej;
-    a.evals[i] =
+    for (int c = 0; c < D; ++c) global_ptr(a.y_final)[c * a.n + i] = L.y[c];
+    global_ptr(a.t_final)[i] = L.t;
+    global_ptr(a.accepted)[i] = L.acc;
+    global_ptr(a.rejected)[i] = L.rej;
+    global_ptr(a.evals)[i] =
         st == kBadInput ? 0 : (int64_t)L.base_ev + 6 * (int64_t)L.rej + 7 * (int64_t)L.acc;
-    a.status[i] = st;
-    if (DENSE && a.n_dense) a.n_dense[i] = L.pushed;
-    if (DENSE && EV == 0 && a.n_pts) a.n_pts[i] = L.pushed;
+    global_ptr(a.status)[i] = st;
+    if (DENSE && a.n_dense) global_ptr(a.n_dense)[i] = L.pushed;
+    if (DENSE && EV == 0 && a.n_pts) global_ptr(a.n_pts)[i] = L.pushed;
     if (DENSE && a.n_eval > 0) teval_tail_nan<D>(a, i, L.next_eval);
     if constexpr (EV != 0) {
       if (a.ev.brk)
@@ -365,14 +367,22 @@ struct Dopri5Lane {
   }
   DE_HD static bool teval_base(const OdeArgs& a) { return EV == 1 && DENSE && a.n_eval > 0; }
   DE_HD static void entry_root(const OdeArgs& a, int64_t i, const double* ent, double* res) {
-    const double tp = ent[kEntryT0], hp = ent[kEntryH];
+    const double tp = global_ptr(ent)[kEntryT0], hp = global_ptr(ent)[kEntryH];
     const double t_new = tp + hp;
-    const double* d = ent + kEntryMeta;
-    double y0p[D], cont1[D], cont2[D], cont3[D];
+    const auto* d = global_ptr(ent) + kEntryMeta;
+    F f;
+    f.load(a.params, a.n, i);
+    double y0p[D], y1p[D], k0p[D], k1p[D], cont1[D], cont2[D], cont3[D];
 #pragma unroll
     for (int c = 0; c < D; ++c) {
-      const double yo = d[c], yn = d[D + c], ko = d[2 * D + c], kn = d[3 * D + c];
-      y0p[c] = yo;
+      y0p[c] = d[c];
+      y1p[c] = d[D + c];
+    }
+    f.diff(tp, y0p, k0p);
+    f.diff(t_new, y1p, k1p);
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      const double yo = y0p[c], yn = y1p[c], ko = k0p[c], kn = k1p[c];
       double ydiff = yn + (-1.0) * yo;
       cont1[c] = ydiff;
       double bspl = hp * ko + (-1.0) * ydiff;
@@ -415,13 +425,13 @@ struct Dopri5Lane {
   DE_HD static double predicted_cost(const OdeArgs& a, int64_t i) {
     F f;
     f.load(a.params, a.n, i);
-    const double t0 = a.t0 ? a.t0[i] : a.t0s;
-    const double tf = a.tf ? a.tf[i] : a.tfs;
+    const double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    const double tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     double h0 = a.h0;
     if (h0 == 0.0 && tf != t0) {
       double y[D];
 #pragma unroll
-      for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+      for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
       LaneTol<D, VTOL> tl;
       tl.load(a, i);
       h0 = lane_h_init(f, t0, tf, y, tl, a.h_min, a.h_max);
@@ -433,11 +443,11 @@ struct Dopri5Lane {
   // (BadInput), after writing its results.
   DE_HD bool init(const OdeArgs& a, int64_t i) {
     f.load(a.params, a.n, i);
-    double t0 = a.t0 ? a.t0[i] : a.t0s;
-    tf = a.tf ? a.tf[i] : a.tfs;
+    double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     tol.load(a, i);
 #pragma unroll
-    for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+    for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
     t = t0;
     acc = rej = 0;
     pushed = 0;
@@ -644,13 +654,11 @@ struct Dopri5Lane {
             bool overflow = false;
             double* ent = ev.defer(a.ev, i, true, tp, hp, tail, pushed, &overflow);
             if (ent) {
-              double* dst = ent + kEntryMeta;
+              auto* dst = global_ptr(ent) + kEntryMeta;
 #pragma unroll
               for (int c = 0; c < D; ++c) {
                 dst[c] = y0p[c];
                 dst[D + c] = ynew[c];
-                dst[2 * D + c] = k0[c];
-                dst[3 * D + c] = dn[c];
               }
             }
             if (overflow) sol = kDeferOverflow;
@@ -737,15 +745,15 @@ struct Dop853Lane {
       }
     }
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.y_final[c * a.n + i] = L.y[c];
-    a.t_final[i] = L.t;
-    a.accepted[i] = L.acc;
-    a.rejected[i] = L.rej;
-    a.evals[i] =
+    for (int c = 0; c < D; ++c) global_ptr(a.y_final)[c * a.n + i] = L.y[c];
+    global_ptr(a.t_final)[i] = L.t;
+    global_ptr(a.accepted)[i] = L.acc;
+    global_ptr(a.rejected)[i] = L.rej;
+    global_ptr(a.evals)[i] =
         st == kBadInput ? 0 : (int64_t)L.base_ev + 11 * (int64_t)(L.acc + L.rej) + 4 * (int64_t)L.acc;
-    a.status[i] = st;
-    if (DENSE && a.n_dense) a.n_dense[i] = L.pushed;
-    if (DENSE && EV == 0 && a.n_pts) a.n_pts[i] = L.pushed;
+    global_ptr(a.status)[i] = st;
+    if (DENSE && a.n_dense) global_ptr(a.n_dense)[i] = L.pushed;
+    if (DENSE && EV == 0 && a.n_pts) global_ptr(a.n_pts)[i] = L.pushed;
     if (DENSE && a.n_eval > 0) teval_tail_nan<D>(a, i, L.next_eval);
     if constexpr (EV != 0) {
       if (a.ev.brk)
@@ -761,10 +769,10 @@ struct Dop853Lane {
     *t1 = ent[kEntryT0] + ent[kEntryH];
   }
   DE_HD static bool entry_interp(const double* ent, double te, double* out) {
-    const double tp = ent[kEntryT0], hp = ent[kEntryH];
+    const double tp = global_ptr(ent)[kEntryT0], hp = global_ptr(ent)[kEntryH];
     const double t_new = tp + hp;
     if (te < tp || te > t_new) return false;
-    const double* d = ent + kEntryMeta;
+    const auto* d = global_ptr(ent) + kEntryMeta;
     const double s = (te - tp) / hp;
     const double s1 = 1.0 - s;
 #pragma unroll
@@ -785,7 +793,7 @@ struct Dop853Lane {
   DE_HD static void entry_root(const OdeArgs& a, int64_t i, const double* ent, double* res) {
     double loc[kEntryWidth];
 #pragma unroll
-    for (int f = 0; f < kEntryWidth; ++f) loc[f] = ent[f];
+    for (int f = 0; f < kEntryWidth; ++f) loc[f] = global_ptr(ent)[f];
     auto interp = [&](double te, double* out) { return entry_interp(loc, te, out); };
     double t0, t1;
     entry_bounds(loc, &t0, &t1);
@@ -810,13 +818,13 @@ struct Dop853Lane {
   DE_HD static double predicted_cost(const OdeArgs& a, int64_t i) {
     F f;
     f.load(a.params, a.n, i);
-    const double t0 = a.t0 ? a.t0[i] : a.t0s;
-    const double tf = a.tf ? a.tf[i] : a.tfs;
+    const double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    const double tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     double h0 = a.h0;
     if (h0 == 0.0 && tf != t0) {
       double y[D];
 #pragma unroll
-      for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+      for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
       LaneTol<D, VTOL> tl;
       tl.load(a, i);
       h0 = lane_h_init<F, LaneTol<D, VTOL>, 8>(f, t0, tf, y, tl, a.h_min, a.h_max);
@@ -826,11 +834,11 @@ struct Dop853Lane {
 
   DE_HD bool init(const OdeArgs& a, int64_t i) {
     f.load(a.params, a.n, i);
-    double t0 = a.t0 ? a.t0[i] : a.t0s;
-    tf = a.tf ? a.tf[i] : a.tfs;
+    double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     tol.load(a, i);
 #pragma unroll
-    for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+    for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
     t = t0;
     acc = rej = 0;
     pushed = 0;
@@ -1120,14 +1128,14 @@ struct FixedLane {
       }
     }
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.y_final[c * a.n + i] = y[c];
-    a.t_final[i] = t;
-    a.accepted[i] = acc;
-    a.rejected[i] = 0;
-    a.evals[i] = ev;
-    a.status[i] = st;
-    if (a.n_dense) a.n_dense[i] = pushed;
-    if (EV == 0 && a.n_pts) a.n_pts[i] = pushed;
+    for (int c = 0; c < D; ++c) global_ptr(a.y_final)[c * a.n + i] = y[c];
+    global_ptr(a.t_final)[i] = t;
+    global_ptr(a.accepted)[i] = acc;
+    global_ptr(a.rejected)[i] = 0;
+    global_ptr(a.evals)[i] = ev;
+    global_ptr(a.status)[i] = st;
+    if (a.n_dense) global_ptr(a.n_dense)[i] = pushed;
+    if (EV == 0 && a.n_pts) global_ptr(a.n_pts)[i] = pushed;
     if (a.n_eval > 0) teval_tail_nan<D>(a, i, next_eval);
     if constexpr (EV != 0) {
       if (a.ev.brk)
@@ -1145,7 +1153,7 @@ struct FixedLane {
   DE_HD static bool entry_interp(const double* ent, double te, double* out) {
     const double tp = ent[kEntryT0], tc = ent[kEntryH];
     if (te < tp || te > tc) return false;
-    const double* d = ent + kEntryMeta;
+    const auto* d = global_ptr(ent) + kEntryMeta;
     double hh = tc - tp;
     double s = (te - tp) / hh;
     double s2 = s * s;
@@ -1164,7 +1172,7 @@ struct FixedLane {
   DE_HD static void entry_root(const OdeArgs& a, int64_t i, const double* ent, double* res) {
     double loc[kEntryWidth];
 #pragma unroll
-    for (int f = 0; f < kEntryWidth; ++f) loc[f] = ent[f];
+    for (int f = 0; f < kEntryWidth; ++f) loc[f] = global_ptr(ent)[f];
     auto interp = [&](double te, double* out) { return entry_interp(loc, te, out); };
     double t0, t1;
     entry_bounds(loc, &t0, &t1);
@@ -1178,18 +1186,18 @@ struct FixedLane {
 
   // Number of steps |tf - t0| / |h0| (only orders work).
   DE_HD static double predicted_cost(const OdeArgs& a, int64_t i) {
-    const double t0 = a.t0 ? a.t0[i] : a.t0s;
-    const double tf = a.tf ? a.tf[i] : a.tfs;
+    const double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    const double tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     const double h0 = a.h0 == 0.0 ? fabs(tf - t0) / 100.0 : a.h0;
     return fabs(tf - t0) / fabs(h0);
   }
 
   DE_HD bool init(const OdeArgs& a, int64_t i) {
     f.load(a.params, a.n, i);
-    double t0 = a.t0 ? a.t0[i] : a.t0s;
-    tf = a.tf ? a.tf[i] : a.tfs;
+    double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
 #pragma unroll
-    for (int c = 0; c < D; ++c) y[c] = a.y0[c * a.n + i];
+    for (int c = 0; c < D; ++c) y[c] = global_ptr(a.y0)[c * a.n + i];
     t = t0;
     acc = ev = 0;
     pushed = 0;
@@ -1299,7 +1307,7 @@ struct FixedLane {
             bool overflow = false;
             double* ent = evs.defer(a.ev, i, true, tp, tc, tail, pushed, &overflow);
             if (ent) {
-              double* dst = ent + kEntryMeta;
+              auto* dst = global_ptr(ent) + kEntryMeta;
 #pragma unroll
               for (int c = 0; c < D; ++c) {
                 dst[c] = yp[c];

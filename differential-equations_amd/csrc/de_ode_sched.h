@@ -77,13 +77,13 @@ ode_persistent_kernel(const OdeArgs* __restrict__ ap) {
         int leader = __ffsll((long long)mask) - 1;
         int cnt = __popcll(mask);
         unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(a.counter, (unsigned long long)cnt);
+        if (lane == leader) base = atomicAdd((unsigned long long*)global_ptr(a.counter), (unsigned long long)cnt);
         base = __shfl(base, leader);
         if (base + (unsigned long long)cnt >= n) drained = true;
         if (need) {
           unsigned long long my = base + (unsigned long long)__popcll(mask & __lanemask_lt());
           if (my < n) {
-            idx = a.order ? (int64_t)a.order[my] : (int64_t)my;
+            idx = a.order ? (int64_t)global_ptr(a.order)[my] : (int64_t)my;
             have = L.begin(a, idx);
           }
         }
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void event_root_kernel(const OdeArgs* __res
   const int t = threadIdx.x;
   const int64_t j0 = (int64_t)blockIdx.x * kBlock;  // position in the slice
   int32_t cnt = 0;
-  if (j0 + t < count) cnt = max(a.ev.bcount[j0 + t], 0);
+  if (j0 + t < count) cnt = max(global_ptr(a.ev.bcount)[j0 + t], 0);
   off[t + 1] = cnt;
   if (t == 0) off[0] = 0;
   __syncthreads();

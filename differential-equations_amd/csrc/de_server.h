@@ -58,6 +58,29 @@ DE_DEV int find_range(const Range* r, int64_t n, int64_t ticket) {
   return (int)lo;
 }
 
+// A slot's part in a chunk: its solver is read and written only while it runs (a
+// pool holds one solver of a few hundred bytes per lane of the device, and few of
+// them run unless the server is loaded).
+template <class L>
+DE_DEV void load_slot(LaneSlot<L>& S, const LaneSlot<L>* slots, int slot, bool valid) {
+  S.state = -1;
+  if (!valid) return;
+  S.ticket = slots[slot].ticket;
+  S.req = slots[slot].req;
+  S.traj = slots[slot].traj;
+  S.state = slots[slot].state;
+  if (S.state == 2) S.s = slots[slot].s;
+}
+template <class L>
+DE_DEV void store_slot(const LaneSlot<L>& S, LaneSlot<L>* slots, int slot, bool valid) {
+  if (!valid) return;
+  slots[slot].ticket = S.ticket;
+  slots[slot].req = S.req;
+  slots[slot].traj = S.traj;
+  slots[slot].state = S.state;
+  if (S.state == 2) slots[slot].s = S.s;
+}
+
 template <class L>
 __global__ __launch_bounds__(kBlock) void chunk_lane(Queue* q, const Range* ranges, ReqDev* reqs,
                                                     LaneSlot<L>* slots, int nslots, int k_iters) {
@@ -65,8 +88,7 @@ __global__ __launch_bounds__(kBlock) void chunk_lane(Queue* q, const Range* rang
   const bool valid = slot < nslots;
   const int lane = __lane_id();
   LaneSlot<L> S;
-  if (valid) S = slots[slot];
-  else S.state = -1;
+  load_slot(S, slots, slot, valid);
   const int64_t published = *(volatile int64_t*)&q->published;
   const int64_t nranges = *(volatile int64_t*)&q->nranges;
   for (int it = 0; it < k_iters; ++it) {
@@ -113,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void chunk_lane(Queue* q, const Range* rang
       S.state = 0;
     }
   }
-  if (valid) slots[slot] = S;
+  store_slot(S, slots, slot, valid);
 }
 
 // Occupancy hints: the rarely taken double-double pow fallback raises the
@@ -129,8 +151,7 @@ chunk_group(Queue* q, const Range* ranges, ReqDev* reqs, LaneSlot<GroupDopri5<G,
   const int l = lane & (G - 1);
   const int leader_lane = lane - l;
   LaneSlot<GroupDopri5<G, C, OUT>> S;
-  if (valid) S = slots[slot];
-  else S.state = -1;
+  load_slot(S, slots, slot, valid);
   const int64_t published = *(volatile int64_t*)&q->published;
   const int64_t nranges = *(volatile int64_t*)&q->nranges;
   for (int it = 0; it < k_iters; ++it) {
@@ -169,7 +190,7 @@ chunk_group(Queue* q, const Range* ranges, ReqDev* reqs, LaneSlot<GroupDopri5<G,
       S.state = 0;
     }
   }
-  if (valid) slots[slot] = S;
+  store_slot(S, slots, slot, valid);
 }
 
 // Reset of a drained pool (no request with work in it): slots that hold an

@@ -89,13 +89,13 @@ struct VecCommon {
       double* yf = a.y_final + A->state_offset[i];
       for (int c = 0; c < n; ++c) yf[c] = y[c];
     }
-    a.t_final[i] = t;
-    a.accepted[i] = acc;
-    a.rejected[i] = rej;
-    a.evals[i] = ev;
-    a.status[i] = st;
-    if (a.n_dense) a.n_dense[i] = pushed;
-    if (a.pts_mode != kPointsNone && a.n_pts) a.n_pts[i] = pushed;
+    global_ptr(a.t_final)[i] = t;
+    global_ptr(a.accepted)[i] = acc;
+    global_ptr(a.rejected)[i] = rej;
+    global_ptr(a.evals)[i] = ev;
+    global_ptr(a.status)[i] = st;
+    if (a.n_dense) global_ptr(a.n_dense)[i] = pushed;
+    if (a.pts_mode != kPointsNone && a.n_pts) global_ptr(a.n_pts)[i] = pushed;
     if (a.n_eval > 0) {  // points not reached (all of them on BadInput)
       double* dbase = a.dense + (int64_t)a.n_eval * A->state_offset[i];
       for (int64_t e = (int64_t)next_eval * n; e < (int64_t)a.n_eval * n; ++e)
@@ -238,15 +238,15 @@ struct VecCommon {
   // The state slot of the next point, or null past this system's slots.
   DE_HD double* pts_dst() const {
     const OdeArgs& a = A->o;
-    return a.pts_offset[i] + pushed < a.pts_offset[i + 1]
+    return global_ptr(a.pts_offset)[i] + pushed < global_ptr(a.pts_offset)[i + 1]
                ? a.pts_y + A->pts_ypos[i] + (int64_t)pushed * n
                : nullptr;
   }
   // Counts the next point and keeps its time while the slots last.
   DE_HD void pts_commit(double tt) {
     const OdeArgs& a = A->o;
-    const int64_t s = a.pts_offset[i] + pushed;
-    if (s < a.pts_offset[i + 1]) a.pts_t[s] = tt;
+    const int64_t s = global_ptr(a.pts_offset)[i] + pushed;
+    if (s < global_ptr(a.pts_offset)[i + 1]) global_ptr(a.pts_t)[s] = tt;
     pushed += 1;
   }
   DE_HD void pts_push(double tt, const double* yy) {
@@ -335,7 +335,7 @@ struct VecCommon {
     double* dbase = a.dense + (int64_t)a.n_eval * A->state_offset[i];
     bool ok = true;
     while (idx < a.n_eval) {
-      double te = a.t_eval[idx];
+      double te = global_ptr(a.t_eval)[idx];
       bool in_range = dir > 0.0 ? ((te == t_prev && idx == 0) || (te > t_prev && te <= t_curr))
                                 : ((te == t_prev && idx == 0) || (te < t_prev && te >= t_curr));
       if (in_range) {
@@ -373,8 +373,8 @@ struct VecCommon {
     y = (A->ystate ? A->ystate : a.y_final) + so;
     const double* y0 = a.y0 + so;
     for (int c = 0; c < n; ++c) y[c] = y0[c];
-    const double t0 = a.t0 ? a.t0[i] : a.t0s;
-    tf = a.tf ? a.tf[i] : a.tfs;
+    const double t0 = a.t0 ? global_ptr(a.t0)[i] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[i] : a.tfs;
     t = t0;
     pushed = next_eval = 0;
     ic0 = 0;
@@ -390,8 +390,8 @@ struct VecCommon {
   DE_HD double h_init(double t0, double* f0, double* f1, double* sk, double* y1) const {
     const OdeArgs& a = A->o;
     const int64_t so = A->state_offset[i];
-    const double rtol = a.rtol_traj ? a.rtol_traj[i] : a.rtol;
-    const double atol = a.atol_traj ? a.atol_traj[i] : a.atol;
+    const double rtol = a.rtol_traj ? global_ptr(a.rtol_traj)[i] : a.rtol;
+    const double atol = a.atol_traj ? global_ptr(a.atol_traj)[i] : a.atol;
     const double* rtv = a.rtol_comp ? a.rtol_comp + so : nullptr;
     const double* atv = a.atol_comp ? a.atol_comp + so : nullptr;
     diff(t0, y, f0);
@@ -446,8 +446,8 @@ struct VecDopri5 : VecCommon {
     for (int v = 0; v < 7; ++v) k[v] = w + (int64_t)v * n;
     ys = w + 7 * (int64_t)n;
     ynew = w + 8 * (int64_t)n;
-    rtol = a.rtol_traj ? a.rtol_traj[i] : a.rtol;
-    atol = a.atol_traj ? a.atol_traj[i] : a.atol;
+    rtol = a.rtol_traj ? global_ptr(a.rtol_traj)[i] : a.rtol;
+    atol = a.atol_traj ? global_ptr(a.atol_traj)[i] : a.atol;
     rtv = a.rtol_comp ? a.rtol_comp + so : nullptr;
     atv = a.atol_comp ? a.atol_comp + so : nullptr;
     acc = rej = ev = steps = 0;
@@ -813,8 +813,8 @@ struct VecDop853 : VecCommon {
     yseg = w + 18 * (int64_t)n;
     cont[0] = y;
     for (int r = 1; r < 8; ++r) cont[r] = w + (int64_t)(18 + r) * n;
-    rtol = a.rtol_traj ? a.rtol_traj[i] : a.rtol;
-    atol = a.atol_traj ? a.atol_traj[i] : a.atol;
+    rtol = a.rtol_traj ? global_ptr(a.rtol_traj)[i] : a.rtol;
+    atol = a.atol_traj ? global_ptr(a.atol_traj)[i] : a.atol;
     rtv = a.rtol_comp ? a.rtol_comp + so : nullptr;
     atv = a.atol_comp ? a.atol_comp + so : nullptr;
     acc = rej = ev = steps = 0;
@@ -1072,8 +1072,8 @@ struct VecErk : VecCommon {
     yh = w + (int64_t)(I + 1) * n;
     dn = w + (int64_t)(I + 2) * n;
     bad = (uint32_t*)(w + (int64_t)(I + 3) * n);
-    rtol = a.rtol_traj ? a.rtol_traj[i] : a.rtol;
-    atol = a.atol_traj ? a.atol_traj[i] : a.atol;
+    rtol = a.rtol_traj ? global_ptr(a.rtol_traj)[i] : a.rtol;
+    atol = a.atol_traj ? global_ptr(a.atol_traj)[i] : a.atol;
     rtv = a.rtol_comp ? a.rtol_comp + so : nullptr;
     atv = a.atol_comp ? a.atol_comp + so : nullptr;
     acc = rej = 0;
@@ -1153,7 +1153,7 @@ struct VecErk : VecCommon {
       else
         interp_out = true;
     } else if (a.n_eval > 0 && accept && next_eval < a.n_eval) {
-      const double te0 = a.t_eval[next_eval];
+      const double te0 = global_ptr(a.t_eval)[next_eval];
       interp_out = !(dir > 0.0 ? te0 > t_new : te0 < t_new);
     }
     if (interp_out || need) {
@@ -1308,8 +1308,8 @@ struct GroupCommon {
 
   // Tolerances of state component c (x_j: c = j, v_j: c = nm + j); the
   // per-component arrays are read where used (their pointer is uniform).
-  DE_DEV double rt(const OdeArgs& a, int c) const { return a.rtol_comp ? a.rtol_comp[so + c] : rtol; }
-  DE_DEV double at(const OdeArgs& a, int c) const { return a.atol_comp ? a.atol_comp[so + c] : atol; }
+  DE_DEV double rt(const OdeArgs& a, int c) const { return a.rtol_comp ? global_ptr(a.rtol_comp)[so + c] : rtol; }
+  DE_DEV double at(const OdeArgs& a, int c) const { return a.atol_comp ? global_ptr(a.atol_comp)[so + c] : atol; }
 
   // Sum of a lane's terms in pairs.  With gsum's levels this is one tree over the
   // mass index for every power-of-two shape (G, C), whose zero terms beyond N add
@@ -1383,8 +1383,8 @@ struct GroupCommon {
     for (int q = 0; q < C; ++q) {
       const int j = l * C + q;
       if (j < nm) {
-        dst[j] = xs[q];
-        dst[nm + j] = vs[q];
+        global_ptr(dst)[j] = xs[q];
+        global_ptr(dst)[nm + j] = vs[q];
       }
     }
   }
@@ -1393,13 +1393,13 @@ struct GroupCommon {
     const OdeArgs& a = A.o;
     write_state(a.y_final + so, x, v);
     if (l == 0) {
-      a.t_final[sys] = t;
-      a.accepted[sys] = acc;
-      a.rejected[sys] = rej;
-      a.evals[sys] = ev;
-      a.status[sys] = st;
-      if (a.n_dense) a.n_dense[sys] = pushed;
-      if (OUT && a.pts_mode != kPointsNone && a.n_pts) a.n_pts[sys] = pushed;
+      global_ptr(a.t_final)[sys] = t;
+      global_ptr(a.accepted)[sys] = acc;
+      global_ptr(a.rejected)[sys] = rej;
+      global_ptr(a.evals)[sys] = ev;
+      global_ptr(a.status)[sys] = st;
+      if (a.n_dense) global_ptr(a.n_dense)[sys] = pushed;
+      if (OUT && a.pts_mode != kPointsNone && a.n_pts) global_ptr(a.n_pts)[sys] = pushed;
     }
     if (a.n_eval > 0) {  // points not reached (all of them on BadInput)
       double nan_[C];
@@ -1537,7 +1537,7 @@ struct GroupCommon {
     double* dbase = a.dense + (int64_t)a.n_eval * so;
     bool ok = true;
     while (idx < a.n_eval) {
-      double te = a.t_eval[idx];
+      double te = global_ptr(a.t_eval)[idx];
       bool in_range = dir > 0.0 ? ((te == t_prev && idx == 0) || (te > t_prev && te <= t_curr))
                                 : ((te == t_prev && idx == 0) || (te < t_prev && te >= t_curr));
       if (in_range) {
@@ -1573,9 +1573,9 @@ struct GroupCommon {
   // state at pts_y[pts_ypos[sys] + k * 2N] while the system's slots last.
   DE_DEV void pts_push(const SpringArgs& A, double tt, const double* xs, const double* vs) {
     const OdeArgs& a = A.o;
-    const int64_t lo = a.pts_offset[sys];
-    if (lo + pushed < a.pts_offset[sys + 1]) {
-      if (l == 0) a.pts_t[lo + pushed] = tt;
+    const int64_t lo = global_ptr(a.pts_offset)[sys];
+    if (lo + pushed < global_ptr(a.pts_offset)[sys + 1]) {
+      if (l == 0) global_ptr(a.pts_t)[lo + pushed] = tt;
       write_state(a.pts_y + A.pts_ypos[sys] + (int64_t)pushed * 2 * nm, xs, vs);
     }
     pushed += 1;
@@ -1653,10 +1653,10 @@ struct GroupCommon {
       x[q] = j < nm ? y0[j] : 0.0;
       v[q] = j < nm ? y0[nm + j] : 0.0;
     }
-    double t0 = a.t0 ? a.t0[s] : a.t0s;
-    tf = a.tf ? a.tf[s] : a.tfs;
-    rtol = a.rtol_traj ? a.rtol_traj[s] : a.rtol;
-    atol = a.atol_traj ? a.atol_traj[s] : a.atol;
+    double t0 = a.t0 ? global_ptr(a.t0)[s] : a.t0s;
+    tf = a.tf ? global_ptr(a.tf)[s] : a.tfs;
+    rtol = a.rtol_traj ? global_ptr(a.rtol_traj)[s] : a.rtol;
+    atol = a.atol_traj ? global_ptr(a.atol_traj)[s] : a.atol;
     t = t0;
     pushed = next_eval = 0;
     ev_count = ev_pushed = 0;
@@ -1681,7 +1681,7 @@ struct GroupCommon {
   // The next t_eval point is not past t_curr (or is NaN): emit has work.
   DE_DEV bool teval_due(const OdeArgs& a, double t_curr) const {
     if (a.n_eval <= 0 || next_eval >= a.n_eval) return false;
-    const double te = a.t_eval[next_eval];
+    const double te = global_ptr(a.t_eval)[next_eval];
     return !(dir > 0.0 ? te > t_curr : te < t_curr);
   }
 };
