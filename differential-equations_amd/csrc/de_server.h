@@ -17,6 +17,7 @@ namespace serve {
 constexpr int kMaxReq = 8192;     // requests resident at once
 constexpr int kMaxRanges = 1 << 20;
 constexpr int kChunk = 256;       // attempts per slot per launch (no backlog)
+constexpr int kQueues = 4;        // hardware queues of a process
 constexpr int kMaxChunk = 4096;   // attempts per slot per launch under a backlog
 constexpr int kBlock = 256;
 
@@ -241,7 +242,7 @@ struct Family {
   int active_reqs = 0;         // active requests with work in this pool
   int64_t max_ranges = 0;      // capacity of the range table
   bool dirty = false;          // published work not yet committed to the device
-  hipStream_t stream = nullptr;
+  int cost = 600;          // of a chunk, relative to the other pools'
   void (*launch)(Family&, ReqDev*, int, hipStream_t) = nullptr;
   void (*reset)(Family&, hipStream_t) = nullptr;
   void (*init)(Family&, hipStream_t) = nullptr;

@@ -199,7 +199,8 @@ struct de_server {
   std::thread thread;
   hipStream_t ctl;
   hipEvent_t fork = nullptr;
-  std::vector<hipEvent_t> fam_done;
+  hipStream_t queue[kQueues] = {};  // the pools' launches, one per hardware queue
+  hipEvent_t queue_done[kQueues] = {};
   hipGraphExec_t graph = nullptr;
   int iterations = 0;
   int64_t range_resets = 0;
@@ -459,16 +460,43 @@ void publish(de_server* s, Family& f, int req_slot, int32_t first, int32_t count
 // slots.
 // With lazy_only, the pools made on first use (outside a captured graph),
 // forked from the event recorded before the graph's launch.
+//
+// A process gets four hardware queues and the kernels of one run one after
+// another, so the iteration lasts as long as its fullest queue.  The pools
+// therefore share four streams: with a short chunk each goes, longest first, to
+// the stream with the least work so far (a stream per pool put Lorenz, 16- and
+// 256-mass chains on one queue: 1.28 of 3.29 ms of kernels in a burst of nine
+// mixed requests); with a backlog's long chunks, where every queue is full, in
+// turn.
 void launch_all(de_server* s, bool busy_only = false, bool lazy_only = false) {
   if (!lazy_only) (void)hipEventRecord(s->fork, s->ctl);
+  std::vector<int> pools;
   for (size_t k = 0; k < s->fams.size(); ++k) {
-    Family& f = s->fams[k];
+    const Family& f = s->fams[k];
     if (!f.slots || (lazy_only && !f.lazy)) continue;
     if (busy_only && f.active_reqs == 0) continue;
-    (void)hipStreamWaitEvent(f.stream, s->fork, 0);
-    f.launch(f, s->d_reqs, s->chunk, f.stream);
-    (void)hipEventRecord(s->fam_done[k], f.stream);
-    (void)hipStreamWaitEvent(s->ctl, s->fam_done[k], 0);
+    pools.push_back((int)k);
+  }
+  const bool balance = s->chunk < kMaxChunk;
+  if (balance)
+    std::stable_sort(pools.begin(), pools.end(), [&](int x, int y) {
+      return s->fams[x].cost > s->fams[y].cost;
+    });
+  int load[kQueues] = {};
+  bool used[kQueues] = {};
+  for (int k : pools) {
+    Family& f = s->fams[k];
+    int q = k % kQueues;
+    if (balance) q = (int)(std::min_element(load, load + kQueues) - load);
+    load[q] += f.cost;
+    if (!used[q]) (void)hipStreamWaitEvent(s->queue[q], s->fork, 0);
+    used[q] = true;
+    f.launch(f, s->d_reqs, s->chunk, s->queue[q]);
+  }
+  for (int q = 0; q < kQueues; ++q) {
+    if (!used[q]) continue;
+    (void)hipEventRecord(s->queue_done[q], s->queue[q]);
+    (void)hipStreamWaitEvent(s->ctl, s->queue_done[q], 0);
   }
 }
 
@@ -494,7 +522,6 @@ bool make_lazy(de_server* s, int k) {
   void* q = slots ? s->arena.alloc(sizeof(Queue)) : nullptr;
   void* ranges = q ? s->arena.alloc(rb) : nullptr;
   bool ok = ranges != nullptr;
-  if (ok && !f.stream) ok = hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) == hipSuccess;
   if (!ok) {
     if (ranges) s->arena.release(ranges, rb);
     if (q) s->arena.release(q, sizeof(Queue));
@@ -747,7 +774,6 @@ bool make_pool(Family& f, int nslots) {
   if (hipMalloc(&f.q, sizeof(de::serve::Queue)) != hipSuccess) return false;
   if (hipMemset(f.q, 0, sizeof(de::serve::Queue)) != hipSuccess) return false;
   if (hipMalloc(&f.ranges, sizeof(Range) * (size_t)f.max_ranges) != hipSuccess) return false;
-  if (hipStreamCreateWithFlags(&f.stream, hipStreamNonBlocking) != hipSuccess) return false;
   return true;
 }
 
@@ -777,14 +803,16 @@ int de_server_create(size_t hbm_budget_bytes, int32_t flags, de_server** out) {
   // the DOP853 lanes of Lorenz and Van der Pol.
   struct Spec {
     const char* name;
-    int cap, g;
+    int cap, g, cost;
   };
-  const Spec specs[] = {{"lorenz", 0, 1},     {"vdp", 0, 1},       {"spring4", 4, 4},
-                        {"spring8", 8, 8},    {"spring16", 16, 16}, {"spring32", 32, 32},
-                        {"spring64", 64, 64}, {"spring128", 128, 64}, {"spring256", 256, 64},
-                        {"lorenz_dop853", 0, 1}, {"vdp_dop853", 0, 1},
-                        {"lorenz_event", 0, 1},  {"lorenz_cross", 0, 1},
-                        {"vdp_event", 0, 1},     {"vdp_cross", 0, 1}};
+  // cost: microseconds of a 256-attempt chunk with few waves per SIMD (the
+  // DOP853 and event lanes by their step's length).
+  const Spec specs[] = {
+      {"lorenz", 0, 1, 540},        {"vdp", 0, 1, 360},          {"spring4", 4, 4, 220},
+      {"spring8", 8, 8, 410},       {"spring16", 16, 16, 280},   {"spring32", 32, 32, 330},
+      {"spring64", 64, 64, 300},    {"spring128", 128, 64, 390}, {"spring256", 256, 64, 460},
+      {"lorenz_dop853", 0, 1, 900}, {"vdp_dop853", 0, 1, 700},   {"lorenz_event", 0, 1, 900},
+      {"lorenz_cross", 0, 1, 900},  {"vdp_event", 0, 1, 700},    {"vdp_cross", 0, 1, 700}};
   static_assert(sizeof specs / sizeof specs[0] == kEagerPools, "pool indices");
   s->fams.resize(kPools);
   const int lane_slots = ncu * 4 * 256;  // 4 blocks of 256 lanes per CU
@@ -803,6 +831,7 @@ int de_server_create(size_t hbm_budget_bytes, int32_t flags, de_server** out) {
     f.name = specs[k].name;
     f.cap = specs[k].cap;
     f.g = specs[k].g;
+    f.cost = specs[k].cost;
     f.max_ranges = max_ranges;
     switch (k) {
       case 0: ok = make_pool<LaneSlot<de::Dopri5Lane<de::LorenzRhs, true>>>(f, lane_slots);
@@ -857,8 +886,10 @@ int de_server_create(size_t hbm_budget_bytes, int32_t flags, de_server** out) {
   s->stage_size = (size_t)64 << 20;
   ok = ok && hipHostMalloc(&s->stage, s->stage_size, 0) == hipSuccess;
   ok = ok && hipEventCreateWithFlags(&s->fork, hipEventDisableTiming) == hipSuccess;
-  s->fam_done.resize(s->fams.size());
-  for (auto& e : s->fam_done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  for (auto& q : s->queue)
+    ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
+  for (auto& e : s->queue_done)
+    ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
   if (ok && hbm_budget_bytes <= pools) ok = false;
   ok = ok && s->arena.init(hbm_budget_bytes - pools, false);
   // Results go to pinned host memory that the kernels write directly, so a
@@ -1084,7 +1115,6 @@ void de_server_destroy(de_server* s) {
       if (f.q) (void)hipFree(f.q);
       if (f.ranges) (void)hipFree(f.ranges);
     }
-    if (f.stream) (void)hipStreamDestroy(f.stream);
   }
   for (auto& kv : s->all) delete kv.second;
   s->arena.destroy();
@@ -1093,13 +1123,15 @@ void de_server_destroy(de_server* s) {
   for (auto h : s->h_counts)
     if (h) (void)hipHostFree(h);
   if (s->d_remaining) (void)hipFree(s->d_remaining);
-  for (auto& e : s->fam_done)
+  for (auto e : s->queue_done)
     if (e) (void)hipEventDestroy(e);
   if (s->fork) (void)hipEventDestroy(s->fork);
   for (auto e : s->ev_counts)
     if (e) (void)hipEventDestroy(e);
   if (s->ev_upl) (void)hipEventDestroy(s->ev_upl);
   if (s->stage) (void)hipHostFree(s->stage);
+  for (auto q : s->queue)
+    if (q) (void)hipStreamDestroy(q);
   if (s->ctl) (void)hipStreamDestroy(s->ctl);
   if (s->upl) (void)hipStreamDestroy(s->upl);
   delete s;
