@@ -88,6 +88,20 @@ DE_HD T* global_ptr(T* p) {
 }
 #endif
 
+// Starts the code after x's computation on a multiple of 8 bytes (one s_nop at most).
+// A double precision instruction is 8 bytes long and is fetched slower where it lies
+// across such a line; a 4-byte one (a move, a compare) shifts all that follow it.  In
+// DOP853's step the run through the stages is long enough to pay: 619 of its 754
+// long instructions lay across a line, 118 do now (3 000 Lorenz trajectories: 1.18 to
+// 1.07 ms, one wave per SIMD; 1 048 576: 33.5 to 31.6).  DOPRI5's (4.17 against
+// 4.21 ms at 1 024 trajectories) and the spring groups' steps (8.87 against 9.52 ms)
+// lose more to the break in their order than they gain.
+#if defined(__HIP_DEVICE_COMPILE__)
+DE_DEV void align_code(double& x) { asm(".p2align 3" : "+v"(x)); }
+#else
+DE_HD void align_code(double&) {}
+#endif
+
 // constrain_step_size (src/utils.rs:22-33): clamp |h| to [h_min, h_max] keeping
 // the sign of h (written with selects; a NaN h is returned unchanged).  signum(h)
 // times a bound is the bound with its sign flipped where h's is set.

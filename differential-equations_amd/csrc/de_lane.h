@@ -896,6 +896,7 @@ struct Dop853Lane {
   DE_HD void stages(double (*k)[D], double* ys) const {
     if constexpr (I < 12) {
       stage_input<I>(y, k, h, ys);
+      align_code(ys[0]);  // 12 stages of some 45 such instructions each
       f.diff(t + d8::C[I] * h, ys, k[I]);
       stages<I + 1>(k, ys);
     }
