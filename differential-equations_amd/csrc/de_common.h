@@ -76,14 +76,23 @@ DE_HD double signum(double x) { return x != x ? x : copysign(1.0, x); }
 // pointers from an argument block in memory, where the compiler only knows generic
 // ones: their accesses would be flat, which count among the scalar loads' waits, so
 // that the next attempt's settings would wait for the last output's store.
+// The caller has to know it: a local array, a member of a lane or LDS as the argument
+// is undefined (a generic address of those is no global one), also where inlining
+// happens to hide it.  Functions that also get a lane's own copy of a record read it
+// plainly.  A host build that defines DE_ON_GLOBAL_PTR(p) sees every argument
+// (tests/cpp/global_ptr_check.cpp).
 #if defined(__HIP_DEVICE_COMPILE__)
 template <class T>
 DE_DEV __attribute__((address_space(1))) T* global_ptr(T* p) {
   return (__attribute__((address_space(1))) T*)p;
 }
 #else
+#if !defined(DE_ON_GLOBAL_PTR)
+#define DE_ON_GLOBAL_PTR(p) ((void)0)
+#endif
 template <class T>
 DE_HD T* global_ptr(T* p) {
+  DE_ON_GLOBAL_PTR(p);
   return p;
 }
 #endif

@@ -768,11 +768,12 @@ struct Dop853Lane {
     *t0 = ent[kEntryT0];
     *t1 = ent[kEntryT0] + ent[kEntryH];
   }
+  // `ent`: the lane's copy of the entry (entry_root's), not global memory.
   DE_HD static bool entry_interp(const double* ent, double te, double* out) {
-    const double tp = global_ptr(ent)[kEntryT0], hp = global_ptr(ent)[kEntryH];
+    const double tp = ent[kEntryT0], hp = ent[kEntryH];
     const double t_new = tp + hp;
     if (te < tp || te > t_new) return false;
-    const auto* d = global_ptr(ent) + kEntryMeta;
+    const double* d = ent + kEntryMeta;
     const double s = (te - tp) / hp;
     const double s1 = 1.0 - s;
 #pragma unroll
@@ -1146,7 +1147,8 @@ struct FixedLane {
     }
   }
 
-  // cubic_hermite_interpolate of a deferred entry, as the step's.
+  // cubic_hermite_interpolate of a deferred entry, as the step's.  `ent`: the
+  // lane's copy of the entry (entry_root's), not global memory.
   DE_HD static void entry_bounds(const double* ent, double* t0, double* t1) {
     *t0 = ent[kEntryT0];
     *t1 = ent[kEntryH];
@@ -1154,7 +1156,7 @@ struct FixedLane {
   DE_HD static bool entry_interp(const double* ent, double te, double* out) {
     const double tp = ent[kEntryT0], tc = ent[kEntryH];
     if (te < tp || te > tc) return false;
-    const auto* d = global_ptr(ent) + kEntryMeta;
+    const double* d = ent + kEntryMeta;
     double hh = tc - tp;
     double s = (te - tp) / hh;
     double s2 = s * s;
