@@ -32,7 +32,7 @@
 // Controller and initial-step pow: the C library's pow that f64::powf calls,
 // restated with the same roundings (de_pow_libm.h) for constant exponents of
 // magnitude below 1/2, in both builds.
-#define DE_CTRL_POW(x, y) ::de::libm_pow_const((x), (y))
+#define DE_CTRL_POW(x, y) DE_POW_CONST(x, y)
 
 namespace de {
 

@@ -1,11 +1,13 @@
 """The controllers' pow (csrc/de_pow_libm.h, libm_pow_const) on the host: the bits
 of libm_pow for every exponent in use, over all regimes of x -- random bit
 patterns (negative, subnormal, NaN), error norms, arguments near 1 (where y log x
-falls below 2^-54), the table's interval ends and the special values."""
+falls below 2^-54), the table's interval ends and the special values.  Exponents
+outside the range whose special cases it leaves out do not compile."""
 import os
 import subprocess
 
 import numpy as np
+import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 EXE = os.path.join(HERE, "cpp", "_build", "pow_check")
@@ -35,3 +37,18 @@ def test_pow_const_has_libm_pow_bits():
     out = subprocess.run([EXE], input=arguments().tobytes(), capture_output=True, timeout=300)
     assert out.returncode == 0, out.stdout.decode()[-2000:]
     assert b", 0 differ" in out.stdout
+
+
+@pytest.mark.parametrize("exponent,takes", [
+    ("-0.2", True), ("1.0 / 9.0", True), ("-(1.0 / 3.0)", True), ("0x1p-10", True),
+    ("0.5", False), ("-0.5", False), ("1.0 / 1.0", False), ("0.0", False), ("0x1p-11", False),
+    ("x", False)])  # x: known at run time only
+def test_exponents_outside_its_range_do_not_compile(exponent, takes):
+    src = ('#include "de_lane.h"\ndouble f(double x) { return DE_CTRL_POW(x, %s); }\n' % exponent)
+    out = subprocess.run(
+        ["g++", "-std=c++17", "-fsyntax-only", "-Wno-unknown-pragmas", "-x", "c++", "-I",
+         os.path.join(HERE, "..", "differential-equations_amd", "csrc"), "-"],
+        input=src, capture_output=True, text=True, timeout=120)
+    assert (out.returncode == 0) == takes, out.stderr[-2000:]
+    if not takes:
+        assert "constant" in out.stderr
