@@ -5,14 +5,11 @@
 
 #include "../../include/de_api.h"
 #include "de_lane.h"
+#include "de_spring_classes.h"
 #include "de_spring_solvers.h"
 
 namespace de {
 namespace parity {
-
-// Size classes: systems of at most kCaps[k] masses.
-constexpr int kCaps[] = {4, 8, 16, 32, 64, 128, 256};
-constexpr int kNumCaps = 7;
 
 typedef void (*GroupKernel)(SpringArgs);
 

@@ -109,59 +109,6 @@ static bool tuned_shape(const Config& cf, int cap) {
   return cf.g * cf.c == cap && cf.g >= 4 && (cf.c < 4 || cap >= 128);
 }
 
-// DOPRI5's size classes: the powers of two and, with three masses per lane, the
-// sizes between them: systems of log-uniform size then fill 85% of their lanes'
-// masses on average (72% with powers of two alone).
-static const int kDopri5Caps[] = {4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256};
-constexpr int kMaxClasses = sizeof(kDopri5Caps) / sizeof(kDopri5Caps[0]);
-static_assert(kNumCaps <= kMaxClasses, "per-class arrays");
-
-// The size classes of a method, and into which class each goes in one launch.
-// Every class is a kernel; those beyond the four hardware queues a process gets
-// wait for one another, and the longest solve bounds each.  So an ensemble whose
-// sizes span more than four classes uses only as many as it has systems for:
-//   few   64 lanes per system, one kernel per number of masses per lane;
-//   mid   (DOPRI5) five classes of 16 to 256 masses;
-//   all   every class.
-// A system keeps its sums' tree (three masses per lane or a power of two) in each
-// of them, so its result does not depend on the ensemble it is in.
-// Measured on chains of 4 to 256 masses, DOPRI5 at rtol 1e-6 over t in [0, 10],
-// few / mid / all in ms: 1024 systems 0.77 / - / 2.16, 4096 1.23 / 1.46 / 2.37,
-// 8192 1.92 / 1.83 / 2.75, 16384 3.44 / 2.62 / 3.44, 32768 6.44 / 4.67 / 4.67,
-// 65536 12.5 / 8.9 / 7.7; RK4 and DOP853, few / all: 1024 0.87 / 1.53 and 0.72 /
-// 1.20, 8192 1.75 / 2.09 and 1.75 / 2.31, 16384 3.19 / 3.14 and 3.16 / 3.23.
-constexpr int kQueues = 4;
-constexpr int64_t kFewSystems = 6144, kMidSystems = 32768;  // DOPRI5
-constexpr int64_t kFewSystemsMethod = 12288;                // the other methods
-enum Merge { kMergeAll = 0, kMergeMid = 1, kMergeFew = 2 };
-
-struct ClassSet {
-  const int* caps;
-  int n;
-};
-static ClassSet class_set(int method) {
-  return method == DE_METHOD_DOPRI5 ? ClassSet{kDopri5Caps, kMaxClasses}
-                                    : ClassSet{kCaps, kNumCaps};
-}
-static Merge merge_of(int method, int64_t systems, int classes) {
-  if (classes <= kQueues) return kMergeAll;
-  if (method != DE_METHOD_DOPRI5) return systems <= kFewSystemsMethod ? kMergeFew : kMergeAll;
-  return systems <= kFewSystems ? kMergeFew : (systems <= kMidSystems ? kMergeMid : kMergeAll);
-}
-// The class that `cap`'s systems are solved in.
-static int merged_cap(Merge m, int cap) {
-  const bool three = cap % 3 == 0;
-  if (m == kMergeFew) return three ? 192 : (cap <= 64 ? 64 : cap);
-  if (m == kMergeMid)
-    return three ? (cap <= 48 ? 48 : 192) : (cap <= 16 ? 16 : (cap <= 64 ? 64 : 256));
-  return cap;
-}
-static int class_index(const ClassSet& cs, int masses) {
-  int k = 0;
-  while (k < cs.n && cs.caps[k] < masses) ++k;
-  return k;
-}
-
 struct Choice {
   int cfg = -1;
   int block = kSpringBlock;
@@ -355,7 +302,8 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   base.list = nullptr;
   base.list_len = 0;
   // Host-side size scan: validity, total state length, classes.
-  const ClassSet cs = class_set(b->method);
+  const bool dopri5 = b->method == DE_METHOD_DOPRI5;
+  const ClassSet cs = class_set(dopri5);
   int64_t state_len = 0;
   std::vector<int64_t> count(cs.n, 0);
   std::vector<uint8_t> class_of((size_t)n);
@@ -406,9 +354,7 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   // Group mapping: the launch's classes, and their lists to upload (one buffer,
   // classes back to back).
   const bool fixed_group = b->mapping == DE_MAP_GROUP && b->group_size > 0;
-  int classes = 0;
-  for (int k = 0; k < cs.n; ++k) classes += count[k] > 0 ? 1 : 0;
-  const Merge merge = fixed_group ? kMergeAll : merge_of(b->method, n, classes);
+  const Merge merge = fixed_group ? kMergeAll : merge_of(dopri5, count.data());
   std::vector<int> merged(cs.n);
   std::vector<int64_t> own = count;
   count.assign(cs.n, 0);
@@ -476,22 +422,24 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
     }
     shape[k] = shape_of(base, ch);
   }
-  // Launch classes concurrently: the three smallest classes first, then the
-  // others largest first.  Every class kernel gets a full-device grid (capped
-  // by its number of systems): the kernels are persistent and exit when their
-  // class is drained, so blocks of the classes launched later are dispatched
-  // as those of earlier ones retire, and the dispatcher balances the classes.
-  // The small classes (N <= 16) hold few waves whose long step sequences set
-  // their time (latency, not throughput): started first, they run beside the
-  // large classes instead of after them, and the largest class then starts
-  // next rather than running alone at the end (measured with seven classes:
-  // 11.8 against 12.7 ms for the 64k-system ensemble, largest first).  (A fixed share per class left the
+  // Launch classes concurrently: every class, smallest first; merged classes, that of up
+  // to 16 masses first, then the others largest first.  Every class kernel gets a
+  // full-device grid (capped by its number of systems): the kernels are persistent and
+  // exit when their class is drained, so blocks of the classes launched later are
+  // dispatched as those of earlier ones retire, and the dispatcher balances the classes.
+  // The small classes hold few waves whose long step sequences set their time (latency,
+  // not throughput): started first, they run beside the large classes (65 536 systems of
+  // 4 to 256 masses, 8.9 against 9.1 ms with only those up to 16 masses before the
+  // rest; 16 384 with 1% above 8 masses 1.44 against 1.65).  One wavefront per system
+  // has no such classes (8192 of 4 to 256 masses with RK4 1.76 ms largest first, 2.09
+  // smallest first).  (A fixed share per class left the
   // GPU idle whenever classes waited behind others for one of the few
   // hardware queues a process gets; ordering each class's systems by size was
   // slower, 14.9 ms: it scatters the group's memory accesses.)
   std::vector<int> launch_order;
-  for (int k = 0; k < cs.n && cs.caps[k] <= 16; ++k) launch_order.push_back(k);
-  for (int k = cs.n - 1; k >= 0 && cs.caps[k] > 16; --k) launch_order.push_back(k);
+  const int ascending = merge == kMergeAll ? 256 : 16;
+  for (int k = 0; k < cs.n && cs.caps[k] <= ascending; ++k) launch_order.push_back(k);
+  for (int k = cs.n - 1; k >= 0 && cs.caps[k] > ascending; --k) launch_order.push_back(k);
   hipLaunchKernelGGL(spring_zero_counters, dim3(1), dim3(64), 0, s, g_counters, cs.n);
   bool ok = hipGetLastError() == hipSuccess && hipEventRecord(g_fork, s) == hipSuccess;
   for (int q = 0; q < cs.n && ok; ++q) {
@@ -502,9 +450,15 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
     ok = hipStreamWaitEvent(g_streams[k], g_fork, 0) == hipSuccess &&
          launch_class(base, d_list + start[k], count[k], share, sh, g_counters + k,
                       g_streams[k]) == 0 &&
-         hipEventRecord(g_join[k], g_streams[k]) == hipSuccess &&
-         hipStreamWaitEvent(s, g_join[k], 0) == hipSuccess;
+         hipEventRecord(g_join[k], g_streams[k]) == hipSuccess;
   }
+  // The caller's stream waits once every class is launched: it shares a hardware queue
+  // with some of the class streams, and a class launched behind one of its waits would
+  // start when another class ends (16 384 chains of 4 to 256 masses with the middle
+  // classes: 2.7 to 3.5 ms, by the queue that the caller's stream has, against 2.5 to
+  // 2.6).
+  for (int k : launch_order)
+    if (ok && count[k] > 0) ok = hipStreamWaitEvent(s, g_join[k], 0) == hipSuccess;
   // The list buffer goes back to the pool after the classes (stream order);
   // the call returns once they are done (the class counters are shared).
   ok = hipFreeAsync(d_list, s) == hipSuccess && ok;

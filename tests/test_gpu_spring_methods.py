@@ -6,6 +6,7 @@ import pytest
 
 import deamd
 from deamd import DE_MAP_AUTO, DE_MAP_GROUP, DE_MAP_LANE, IVP, ExplicitRungeKutta, SpringChain
+from test_spring_classes import classes_of
 
 pytestmark = pytest.mark.gpu
 
@@ -104,15 +105,14 @@ def test_values_that_overflow(orc, method):
     check(orc, ens, (DE_MAP_AUTO, DE_MAP_LANE))
 
 
-@pytest.mark.parametrize("method,sizes", [("dopri5", (300, 6144, 6145, 32768, 32769)),
-                                          ("dop853", (300, 12288, 12289)),
-                                          ("rk4", (300, 12289))])
+@pytest.mark.parametrize("method,sizes", [("dopri5", (300, 6144, 6145, 16384)),
+                                          ("dop853", (300, 12289)), ("rk4", (300, 12289))])
 def test_results_do_not_depend_on_the_batch(orc, method, sizes):
-    # The classes that a launch uses follow the number of systems; a system has
-    # the same bits alone, in a small ensemble and on either side of each rule.
+    # The classes that a launch uses follow its systems; a system has the same bits
+    # alone and in an ensemble of every set of classes.
     edges = [6, 23, 40, 100, 160, 200, 3, 64]
     rng = np.random.default_rng(75)
-    pool = np.concatenate([edges, rng.integers(1, 257, 92)])
+    pool = np.concatenate([edges, rng.integers(1, 33, 92)])
     sysm, y0 = chains(pool, 75)
 
     def part(idx):
@@ -124,12 +124,15 @@ def test_results_do_not_depend_on_the_batch(orc, method, sizes):
     alone = [part([i]).solve() for i in range(len(edges))]
     if method != "dopri5":
         assert all(np.array_equal(a.y, orc.solve_ode(part([i])).y) for i, a in enumerate(alone))
+    sets = set()
     for n in sizes:
         idx = np.concatenate([np.arange(len(edges)), rng.integers(0, len(pool), n - len(edges))])
+        sets.add(classes_of(method == "dopri5", pool[idx]))
         whole = part(idx).solve()
         for i, one in enumerate(alone):
             assert np.array_equal(one.y, whole.final_state(i)), (n, i)
             assert one.accepted[0] == whole.accepted[i] and one.evals[0] == whole.evals[i]
+    assert sets == ({"few", "mid", "all"} if method == "dopri5" else {"few", "all"})
 
 
 @pytest.mark.parametrize("out", ["final", "t_eval", "points", "event"])
