@@ -113,5 +113,21 @@ inline Merge merge_of(bool dopri5, const int64_t* count) {
   return best;
 }
 
+// DOPRI5's shape for a caller's number of lanes per system (a power of two up to 64) in
+// the class of `cap` masses: that many lanes where 1, 2 or 4 masses per lane fill the
+// class, or where 3 hold it in a class of three masses per lane; otherwise the class's
+// shape of most masses per lane.  Lanes beyond a class of three masses per lane add
+// zeros, so the sums keep their tree.
+struct LaneShape {
+  int g, c;
+};
+inline LaneShape group_shape(int cap, int lanes) {
+  const bool power = lanes >= 1 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
+  if (cap % 3 == 0) return {power && lanes * 3 >= cap ? lanes : cap / 3, 3};
+  for (int c = 1; c <= 4; c *= 2)
+    if (power && lanes * c == cap) return {lanes, c};
+  return {cap / 4, 4};
+}
+
 }  // namespace parity
 }  // namespace de

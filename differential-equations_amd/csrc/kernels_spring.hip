@@ -189,12 +189,17 @@ static int launch_class(const SpringArgs& base, const int32_t* d_list, int64_t l
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+static int config_of(const LaneShape& sh) {
+  for (int ci = 0; ci < kNumConfigs; ++ci)
+    if (kConfigs[ci].g == sh.g && kConfigs[ci].c == sh.c) return ci;
+  return -1;
+}
+
 // The shape of 64 lanes for `cap` masses.
 static Choice wave_per_system(int cap) {
   Choice ch;
   ch.block = kTunedBlock;
-  for (int ci = 0; ci < kNumConfigs; ++ci)
-    if (kConfigs[ci].g == 64 && 64 * kConfigs[ci].c == cap) ch.cfg = ci;
+  ch.cfg = config_of({64, cap / 64});
   return ch;
 }
 
@@ -395,16 +400,7 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
     }
     Choice ch;
     if (fixed_group) {
-      for (int ci = 0; ci < kNumConfigs; ++ci)
-        if (kConfigs[ci].g == b->group_size && kConfigs[ci].g * kConfigs[ci].c == cs.caps[k])
-          ch.cfg = ci;
-      if (ch.cfg < 0) {
-        // group size too small for this class: largest C that covers the cap
-        for (int ci = 0; ci < kNumConfigs; ++ci)
-          if (kConfigs[ci].g * kConfigs[ci].c == cs.caps[k] &&
-              (ch.cfg < 0 || kConfigs[ci].c > kConfigs[ch.cfg].c))
-            ch.cfg = ci;
-      }
+      ch.cfg = config_of(group_shape(cs.caps[k], b->group_size));
     } else {
       if (merge == kMergeFew) {
         ch = wave_per_system(cs.caps[k]);
@@ -415,10 +411,10 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
         if (known.cfg < 0) known = autotune(base, cs.caps[k], d_list + start[k], count[k], s);
         ch = known;
       }
-      if (ch.cfg < 0) {
-        (void)hipFreeAsync(d_list, s);
-        return -1;
-      }
+    }
+    if (ch.cfg < 0) {
+      (void)hipFreeAsync(d_list, s);
+      return -1;
     }
     shape[k] = shape_of(base, ch);
   }

@@ -109,7 +109,11 @@ extern "C" {
 /* Mappings of a system onto lanes (spring chain). */
 #define DE_MAP_AUTO 0  /* autotuner picks per size class */
 #define DE_MAP_LANE 1  /* one lane per system, state in HBM */
-#define DE_MAP_GROUP 2 /* `group_size` lanes per system, state in registers */
+#define DE_MAP_GROUP 2 /* `group_size` lanes per system, state in registers.  DOPRI5: a power
+                          of two up to 64, taken where the system has at least that many
+                          masses and at most four per lane; otherwise its size class's own
+                          shape.  The other methods have one shape per size class.  The
+                          shape does not change a system's result. */
 
 /* Solouts beside DefaultSolout / TEvalSolout (src/solout, builders src/ivp.rs:662-705). */
 #define DE_SOLOUT_DEFAULT 0    /* DefaultSolout, or TEvalSolout when n_eval > 0 */

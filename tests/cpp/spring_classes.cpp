@@ -1,6 +1,7 @@
 // The spring chains' class rules (csrc/de_spring_classes.h) on the host.  Reads lines
 // "dopri5 n size count size count ..." and prints the set of classes that a launch of
-// those systems uses.
+// those systems uses; "shape masses lanes" prints the lanes and masses per lane of
+// DE_MAP_GROUP with that group_size.
 #include <stdio.h>
 
 #include <sstream>
@@ -15,6 +16,15 @@ using namespace de::parity;
 int main() {
   for (std::string line; std::getline(std::cin, line);) {
     std::istringstream in(line);
+    if (line.rfind("shape", 0) == 0) {
+      std::string word;
+      int masses = 0, lanes = 0;
+      in >> word >> masses >> lanes;
+      const ClassSet cs = class_set(true);
+      const LaneShape sh = group_shape(cs.caps[class_index(cs, masses)], lanes);
+      printf("%d %d\n", sh.g, sh.c);
+      continue;
+    }
     int dopri5 = 0, size = 0;
     long long n = 0;
     in >> dopri5;

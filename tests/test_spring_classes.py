@@ -75,3 +75,14 @@ def test_no_more_classes_than_queues_use_their_own(sizes):
     for n in (1, 100, 100000):
         assert [r[0] for r in run([line(d, np.repeat(sizes, n)) for d in (True, False)])] == \
             ["all", "all"]
+
+
+def test_a_callers_group_size_is_taken():
+    # Every chain of at least as many masses as lanes and at most four per lane gets the
+    # lanes asked for; the others a shape that holds them.
+    asked = [(n, g) for n in range(1, 257) for g in (1, 2, 4, 8, 16, 32, 64)]
+    got = [tuple(map(int, r)) for r in run(["shape %d %d" % a for a in asked])]
+    for (n, lanes), (g, c) in zip(asked, got):
+        assert g * c >= n and c in (1, 2, 3, 4) and g <= 64
+        if lanes <= n <= 4 * lanes:
+            assert g == lanes, (n, lanes, g, c)
