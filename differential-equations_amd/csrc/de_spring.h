@@ -31,8 +31,8 @@ DE_SPRING_PARTS(DE_SPRING_PART_DECL)
 int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArgs& a, int sched,
                   hipStream_t s);
 int64_t spring_workspace_bytes(const de_ode_batch* b);
-// The library's shape for the size class with cap masses: 0 and (G, C, block), or
-// -1 if none of its systems has been solved in this process.
+// The shape (G, C, block) that the systems of the size class with cap masses were last
+// solved with: 0, or -1 if none has been solved with a shape of the library's choice.
 int spring_tuned(int cap, int* g, int* c, int* block);
 
 }  // namespace parity

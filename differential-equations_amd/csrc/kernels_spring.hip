@@ -122,11 +122,12 @@ struct Shape {
 
 // Process-wide state: autotune decisions per size class, streams, workspace.
 static std::mutex g_mu;
-// DOPRI5's choices by class cap: the autotuner's, for ensembles that use every class
-// and for those that use five, and the caps solved with 64 lanes per system.
-// Which shape is picked does not change a system's result.
+// DOPRI5's shapes of the library's choice by class cap: the autotuner's, for ensembles
+// that use every class and for those that use five, and the one that each class's
+// systems were last solved with.  Which shape is picked does not change a system's
+// result.
 static std::map<int, Choice> g_tuned[2];
-static std::map<int, Choice> g_few;
+static std::map<int, Choice> g_solved;
 static hipStream_t g_streams[kMaxClasses] = {};
 static hipEvent_t g_fork = nullptr, g_join[kMaxClasses] = {};
 static unsigned long long* g_counters = nullptr;
@@ -404,13 +405,13 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
     } else {
       if (merge == kMergeFew) {
         ch = wave_per_system(cs.caps[k]);
-        for (int o = 0; o < cs.n; ++o)
-          if (merged[o] == k && own[o] > 0) g_few[cs.caps[o]] = ch;
       } else {
         Choice& known = g_tuned[merge][cs.caps[k]];
         if (known.cfg < 0) known = autotune(base, cs.caps[k], d_list + start[k], count[k], s);
         ch = known;
       }
+      for (int o = 0; o < cs.n; ++o)
+        if (merged[o] == k && own[o] > 0) g_solved[cs.caps[o]] = ch;
     }
     if (ch.cfg < 0) {
       (void)hipFreeAsync(d_list, s);
@@ -462,24 +463,15 @@ int launch_spring(const de_ode_batch* b, const int32_t* host_sizes, const OdeArg
   return ok ? 0 : -1;
 }
 
-// Introspection: the shape (G, C, block) of the size class of `cap` masses, or -1
-// if none of its systems has been solved with a shape of the library's choice.
-// Where a class was only solved with 64 lanes per system, G is the number of those
-// that hold its masses.
+// Introspection: the shape (G, C, block) that the systems of the size class of `cap`
+// masses were last solved with, or -1 if none has been solved with a shape of the
+// library's choice.
 int spring_tuned(int cap, int* g, int* c, int* block) {
   std::lock_guard<std::mutex> lk(g_mu);
-  for (const auto& tuned : g_tuned) {
-    auto it = tuned.find(cap);
-    if (it == tuned.end() || it->second.cfg < 0) continue;
-    *g = kConfigs[it->second.cfg].g;
-    *c = kConfigs[it->second.cfg].c;
-    *block = it->second.block;
-    return 0;
-  }
-  auto it = g_few.find(cap);
-  if (it == g_few.end()) return -1;
+  auto it = g_solved.find(cap);
+  if (it == g_solved.end() || it->second.cfg < 0) return -1;
+  *g = kConfigs[it->second.cfg].g;
   *c = kConfigs[it->second.cfg].c;
-  *g = cap / *c;
   *block = it->second.block;
   return 0;
 }

@@ -65,9 +65,12 @@ int de_diag_fmt(const double* x, char* out, int32_t* len, int64_t n);
 int de_diag_noise(uint64_t seed, const uint64_t* path, const uint32_t* step,
                   const uint32_t* comp, double* out, int64_t n);
 
-/* Spring-chain autotuner decision for the size class whose largest chain has
- * `cap` masses (4, 8, ..., 256): lanes per system G, masses per lane C and
- * block size.  Returns 0, or -1 if the class has not been tuned yet. */
+/* Shape in which DOPRI5 spring chains of the size class whose largest chain has `cap`
+ * masses (4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256) were last solved by the library's
+ * choice (DE_MAP_AUTO, or DE_MAP_GROUP without a group_size): lanes per system G, masses
+ * per lane C and block size.  G * C is `cap` where the class was launched by itself (the
+ * autotuner's choice among its shapes), and larger where the launch solved it with
+ * larger classes.  Returns 0, or -1 if no such system has been solved yet. */
 int de_spring_tuned(int32_t cap, int32_t* g, int32_t* c, int32_t* block);
 
 #ifdef __cplusplus

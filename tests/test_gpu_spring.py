@@ -68,17 +68,55 @@ def test_group_mappings_within_bound(case, mapping, group):
     assert dense_err <= 1e-9, dense_err
 
 
-def test_autotuner_reports_its_choices(case):
-    sysm, ens, want = case
-    ens.options(mapping=DE_MAP_AUTO).solve()
+CAPS = (4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)
+
+
+def tuned(cap):
     import ctypes as C
-    lib = deamd.lib()
-    caps = sorted({c for c in (4, 8, 16, 32, 64, 128, 256)
-                   if ((sysm.sizes <= c) & (sysm.sizes > c // 2 if c > 4 else True)).any()})
+    g, c, b = C.c_int32(), C.c_int32(), C.c_int32()
+    rc = deamd.lib().de_spring_tuned(cap, C.byref(g), C.byref(c), C.byref(b))
+    return (g.value, c.value, b.value) if rc == 0 else None
+
+
+@pytest.mark.parametrize("caps", [CAPS[:4], CAPS[4:8], CAPS[8:]])
+def test_autotuner_reports_its_choices(caps):
+    # No more than four classes: each is launched by itself, in one of the shapes
+    # that the autotuner times.
+    rng = np.random.default_rng(caps[0])
+    lo = [0] + list(CAPS)
+    sizes = np.concatenate([rng.integers(lo[CAPS.index(c)] + 1, c + 1, 60) for c in caps])
+    sizes = sizes.astype(np.int32)
+    p = np.concatenate([np.r_[0.05, np.ones(n + 1)] for n in sizes])
+    ens = IVP.ode(deamd.SpringChain(sizes, p), 0.0, 1.0,
+                  rng.standard_normal(int(2 * sizes.sum()))).method(
+        ExplicitRungeKutta.dopri5().rtol(1e-6).atol(1e-9))
+    ens.options(mapping=DE_MAP_AUTO).solve()
     for cap in caps:
-        g, c, b = C.c_int32(), C.c_int32(), C.c_int32()
-        assert lib.de_spring_tuned(cap, C.byref(g), C.byref(c), C.byref(b)) == 0
-        assert g.value * c.value == cap and b.value in (64, 256)
+        g, c, b = tuned(cap)
+        assert g * c == cap and b in (64, 256)
+        assert g >= 4 and c <= (4 if cap >= 128 else 3)
+
+
+@pytest.mark.parametrize("n,sets", [(2048, "few"), (8192, "mid")])
+def test_shapes_of_merged_classes_are_reported(n, sets):
+    # Every class with systems is reported with the shape that was launched.
+    from test_spring_classes import classes_of
+    sysm, y0 = deamd.gen_spring(n, seed=17)
+    assert classes_of(True, sysm.sizes) == sets
+    IVP.ode(sysm, 0.0, 1.0, y0).method(ExplicitRungeKutta.dopri5().rtol(1e-6).atol(1e-9)) \
+        .options(mapping=DE_MAP_AUTO).solve()
+    present = [c for lo, c in zip((0,) + CAPS, CAPS)
+               if ((sysm.sizes > lo) & (sysm.sizes <= c)).any()]
+    assert len(present) > 4
+    for cap in present:
+        g, c, b = tuned(cap)
+        three = cap % 3 == 0
+        if sets == "few":
+            assert (g, c) == (64, 3 if three else max(cap // 64, 1)), cap
+        else:
+            merged = (48 if cap <= 48 else 192) if three else min(
+                m for m in (16, 64, 256) if m >= cap)
+            assert g * c == merged, cap
 
 
 def test_mixed_sizes_results_do_not_depend_on_batch_composition(case):
