@@ -12,7 +12,8 @@
  * thread-local message readable with de_last_error().
  *
  * Memory: by default every pointer is device memory (HBM) and the call is
- * asynchronous on `stream` (a hipStream_t, NULL = default stream).  With
+ * asynchronous on `stream` (a hipStream_t, NULL = default stream; spring chains'
+ * sizes are read back first, so what wrote them must have ended).  With
  * DE_FLAG_HOST_MEMORY every pointer is host memory; the library stages copies
  * and returns after the results are back on the host.
  *
