@@ -228,7 +228,7 @@ DE_HD double libm_pow(double x, double y) {
 }
 
 // The exponents of libm_pow_const.
-constexpr bool pow_const_takes(double y) {
+DE_HD constexpr bool pow_const_takes(double y) {
   return (y < 0.0 ? -y : y) >= 0x1p-10 && (y < 0.0 ? -y : y) < 0.5;
 }
 template <bool TAKEN>

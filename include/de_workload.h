@@ -53,7 +53,8 @@ void de_philox4x32_10(const uint32_t ctr[4], uint32_t k0, uint32_t k1, uint32_t 
 double de_noise_normal(uint64_t seed, uint64_t path, uint32_t step, uint32_t comp);
 
 /* Device self-checks (run on the GPU, compare with the host in tests):
- * out[i] = pow(x[i], y[i]) with the integrator's pow; x/y/out host memory. */
+ * out[i] = pow(x[i], y[i]) with the integrator's pow (for 2^-10 <= |y| < 1/2 the form
+ * that the step size controllers use); x/y/out host memory. */
 int de_diag_pow(const double* x, const double* y, double* out, int64_t n);
 /* out[3*i + 0..2] = a/b, sqrt(a), fma(a, b, c) as computed on the device. */
 int de_diag_arith(const double* a, const double* b, const double* c, double* out,

@@ -1,5 +1,5 @@
-"""The controllers' pow (csrc/de_pow_libm.h, libm_pow_const) on the host: the bits
-of libm_pow for every exponent in use, over all regimes of x -- random bit
+"""The controllers' pow (csrc/de_pow_libm.h, libm_pow_const), built for the host and
+in the device library: the bits of libm_pow for every exponent in use, over all regimes of x -- random bit
 patterns (negative, subnormal, NaN), error norms, arguments near 1 (where y log x
 falls below 2^-54), the table's interval ends and the special values.  Exponents
 outside the range whose special cases it leaves out do not compile."""
@@ -32,8 +32,7 @@ def arguments():
 
 
 def test_pow_const_has_libm_pow_bits():
-    if not os.path.exists(EXE):
-        subprocess.check_call(["make", "-s", "-C", os.path.join(HERE, "cpp"), "_build/pow_check"])
+    subprocess.check_call(["make", "-s", "-C", os.path.join(HERE, "cpp"), "_build/pow_check"])
     out = subprocess.run([EXE], input=arguments().tobytes(), capture_output=True, timeout=300)
     assert out.returncode == 0, out.stdout.decode()[-2000:]
     assert b", 0 differ" in out.stdout
@@ -52,3 +51,17 @@ def test_exponents_outside_its_range_do_not_compile(exponent, takes):
     assert (out.returncode == 0) == takes, out.stderr[-2000:]
     if not takes:
         assert "constant" in out.stderr
+
+
+@pytest.mark.gpu
+def test_device_build_has_the_host_bits(orc):
+    import deamd
+    x = arguments()
+    for y in [-0.2, 0.2, -0.125, 0.125] + [s / k for k in (4, 6, 7, 9) for s in (-1.0, 1.0)] + \
+            [2.0 ** -10, -0.499]:
+        ys, out = np.full_like(x, y), np.empty_like(x)
+        deamd._abi.check(deamd.lib().de_diag_pow(deamd._ptr(x), deamd._ptr(ys),
+                                                 deamd._ptr(out), len(x)))
+        want = orc.pow_many(x, ys)
+        assert ((out.view(np.uint64) == want.view(np.uint64)) |
+                (np.isnan(out) & np.isnan(want))).all(), y
