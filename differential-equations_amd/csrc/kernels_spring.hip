@@ -7,13 +7,14 @@
 //                 DOPRI5 to rounding (its norm is summed over the lanes); the
 //                 other methods keep the one-lane solvers' bits and have one
 //                 shape per size class (kernels_spring_group.hip).
-//   DE_MAP_AUTO   as DE_MAP_GROUP.  Systems are bucketed into size classes
-//                 (N <= 4, 8, ..., 256);
-//                 for each class of DOPRI5 an autotuner times the shapes (G, C)
-//                 with G*C equal to the class cap on a sample of the class and
-//                 keeps the fastest.  Classes run concurrently on their own streams,
-//                 each as a persistent kernel whose groups take the next system
-//                 of the class from a work counter when they finish one.
+//   DE_MAP_AUTO   as DE_MAP_GROUP without a group_size.  Systems are bucketed into
+//                 size classes, some of which a launch may merge
+//                 (de_spring_classes.h); for each class of DOPRI5 an autotuner
+//                 times the shapes (G, C) with G*C equal to the class cap on a
+//                 sample of the class and keeps the fastest.  Classes run
+//                 concurrently on their own streams, each as a persistent kernel
+//                 whose groups take the next system of the class from a work
+//                 counter when they finish one.
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -258,6 +259,9 @@ static Choice autotune(const SpringArgs& base, int cap, const int32_t* d_list, i
       candidates += 1;
     }
   if (candidates <= 1) return best;
+  // Solves of other streams still run: their classes would lengthen some of the times.
+  for (hipStream_t other : g_streams)
+    if (hipStreamSynchronize(other) != hipSuccess) return best;
   best.cfg = -1;
   float best_ms = 1e30f;
   const int64_t sample = len < 8192 ? len : 8192;
