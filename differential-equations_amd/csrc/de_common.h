@@ -102,7 +102,8 @@ DE_HD T* global_ptr(T* p) {
 // across such a line; a 4-byte one (a move, a compare) shifts all that follow it.  In
 // DOP853's step the run through the stages is long enough to pay: 619 of its 754
 // long instructions lay across a line, 118 do now (3 000 Lorenz trajectories: 1.18 to
-// 1.07 ms, one wave per SIMD; 1 048 576: 33.5 to 31.6).  DOPRI5's (4.17 against
+// 1.07 ms, one wave per SIMD; 1 048 576: 33.5 to 31.6, the time from before the outputs
+// became global stores, which had moved the run by four bytes).  DOPRI5's (4.17 against
 // 4.21 ms at 1 024 trajectories) and the spring groups' steps (8.87 against 9.52 ms)
 // lose more to the break in their order than they gain.
 #if defined(__HIP_DEVICE_COMPILE__)
